@@ -19,6 +19,7 @@ struct FilterStage {
   int project = 0;
   double beta = 1.0, eta = 0.5;
   DeviceBuffer wt, rx;   // cone weights and per-(dz, dy) x extents
+  DeviceBuffer wd2;      // the weights by squared offset
   DeviceBuffer den;      // W 1 (rows outside the box: 1)
   DeviceBuffer dens;     // density-filtered field of the last design call
   DeviceBuffer proj;     // projected field of the last design call (projecting stages)
@@ -34,7 +35,7 @@ struct Filter {
   int fbox[6], dbox[6];
   hipStream_t own = nullptr;
   hipEvent_t ev[2] = {nullptr, nullptr};
-  DeviceBuffer background, design_in, full0, tmp, acc, design_out;
+  DeviceBuffer background, design_in, tmp, acc, design_out;
   std::vector<std::unique_ptr<FilterStage>> stages;
   bool have_design = false;
   double ms[2] = {0, 0};
@@ -68,7 +69,6 @@ struct Filter {
     HIP_OK(hipEventCreate(&ev[1]));
     const size_t nb = (size_t)N * 8;
     background.ensure(nb);
-    full0.ensure(nb);
     tmp.ensure(nb);
     acc.ensure(nb);
     design_in.ensure((size_t)ND * 8);
@@ -119,6 +119,10 @@ struct Filter {
             r = std::max(r, std::abs(dx));
           }
         }
+    std::vector<double> wd2((size_t)R * R + 1);
+    for (int d2 = 0; d2 <= R * R; ++d2) wd2[d2] = fr - std::sqrt((double)d2);
+    st.wd2.ensure(wd2.size() * 8);
+    HIP_OK(hipMemcpy(st.wd2.p, wd2.data(), wd2.size() * 8, hipMemcpyHostToDevice));
     st.wt.ensure(wt.size() * 8);
     st.rx.ensure(rx.size() * sizeof(int));
     HIP_OK(hipMemcpy(st.wt.p, wt.data(), wt.size() * 8, hipMemcpyHostToDevice));
@@ -131,41 +135,55 @@ struct Filter {
     a.out = out;
     a.den = st.den.as<double>();
     a.wt = st.wt.as<double>();
+    a.wd2 = st.wd2.as<double>();
     a.rx = st.rx.as<int>();
     a.nx = d.nx;
     a.ny = d.ny;
     a.nz = d.nz;
     a.R = st.R;
-    for (int k = 0; k < 6; ++k) a.box[k] = fbox[k];
+    for (int k = 0; k < 6; ++k) {
+      a.box[k] = fbox[k];
+      a.dbox[k] = dbox[k];
+    }
     a.transposed = transposed ? 1 : 0;
     return a;
   }
 
-  // tanh(beta eta) and tanh(beta eta) + tanh(beta (1 - eta)) of a projecting stage
-  static void proj_consts(const FilterStage& st, double& tb, double& tsum) {
-    tb = std::tanh(st.beta * st.eta);
-    tsum = tb + std::tanh(st.beta * (1.0 - st.eta));
+  // tanh(beta eta) and tanh(beta eta) + tanh(beta (1 - eta)) of a projecting stage with its eta
+  static ProjectArgs projection(const FilterStage& st) {
+    ProjectArgs p{};
+    p.on = st.project;
+    p.beta = st.beta;
+    p.eta = st.eta;
+    p.tb = std::tanh(st.beta * st.eta);
+    p.tsum = p.tb + std::tanh(st.beta * (1.0 - st.eta));
+    p.etaf = st.eta_field();
+    return p;
   }
 
   // mapDesignToFull + filterDesign of every stage (the last stage's output is the physical
-  // field); the design is a host array, or a device array read in place when dev is set
-  const double* run_design(const double* design, bool dev, hipStream_t s) {
+  // field), one launch per stage: the first reads the design and the background in place of
+  // the mapped field, each projects its own output, the last also writes `physical` (a device
+  // array, or nullptr). The design is a host array, or a device array read in place when dev
+  // is set.
+  const double* run_design(const double* design, bool dev, double* physical, hipStream_t s) {
     const double* din = design;
     if (!dev) {
       HIP_OK(hipMemcpyAsync(design_in.p, design, (size_t)ND * 8, hipMemcpyHostToDevice, s));
       din = design_in.as<double>();
     }
     HIP_OK(hipEventRecord(ev[0], s));
-    HIP_OK(launch_map_to_full(full0.as<double>(), din, background.as<double>(), d.nx, d.ny, d.nz, dbox, s));
-    const double* x = full0.as<double>();
+    const double* x = nullptr;
     for (auto& st : stages) {
-      HIP_OK(launch_cone(cone_args(*st, x, st->dens.as<double>(), false), s));
-      if (st->project) {
-        double tb, tsum;
-        proj_consts(*st, tb, tsum);
-        HIP_OK(launch_project(st->proj.as<double>(), st->dens.as<double>(), d.nx, d.ny, d.nz, fbox, st->beta,
-                              st->eta, tb, tsum, st->eta_field(), s));
+      ConeArgs a = cone_args(*st, x, st->dens.as<double>(), false);
+      if (!x) {
+        a.design = din;
+        a.background = background.as<double>();
       }
+      a.proj = projection(*st);
+      if (st->project) a.proj_out = st->proj.as<double>();
+      if (st == stages.back()) a.copy_out = physical;
+      HIP_OK(launch_cone(a, s));
       x = st->output();
     }
     HIP_OK(hipEventRecord(ev[1], s));
@@ -174,23 +192,31 @@ struct Filter {
   }
 
   // filterSensitivities (stages in reverse) + mapFullToDesign; sens_dev is only read. The
-  // result goes to a host array, or straight into a device array when out_dev is set.
+  // result goes to a host array, or straight into a device array when out_dev is set. Each
+  // transposed filter hands its result on already scaled for the stage before it; the first
+  // stage's writes the design box alone.
   void run_sensitivities(const double* sens_dev, double* out, bool out_dev, hipStream_t s) {
     for (auto& st : stages)
       if (st->project && !have_design)
         throw Error{LBMX_ERR_STATE, "a projecting filter needs lbmx_filter_design before its sensitivities"};
     HIP_OK(hipEventRecord(ev[0], s));
-    const double* cur = sens_dev;
-    for (int k = (int)stages.size() - 1; k >= 0; --k) {
-      FilterStage& st = *stages[k];
-      double tb = 0, tsum = 1;
-      if (st.project) proj_consts(st, tb, tsum);
-      HIP_OK(launch_sens_scale(tmp.as<double>(), cur, st.dens.as<double>(), st.den.as<double>(), d.nx, d.ny, d.nz,
-                               fbox, st.project, st.beta, st.eta, tsum, st.eta_field(), s));
-      HIP_OK(launch_cone(cone_args(st, tmp.as<double>(), acc.as<double>(), true), s));
-      cur = acc.as<double>();
+    const int last = (int)stages.size() - 1;
+    double* cur = tmp.as<double>();
+    double* next = acc.as<double>();
+    HIP_OK(launch_sens_scale(cur, sens_dev, stages[last]->dens.as<double>(), stages[last]->den.as<double>(), d.nx,
+                             d.ny, d.nz, fbox, projection(*stages[last]), s));
+    for (int k = last; k >= 0; --k) {
+      ConeArgs a = cone_args(*stages[k], cur, next, true);
+      if (k == 0) {
+        a.design_out = out_dev ? out : design_out.as<double>();
+      } else {
+        a.proj = projection(*stages[k - 1]);
+        a.scale_x = stages[k - 1]->dens.as<double>();
+        a.scale_den = stages[k - 1]->den.as<double>();
+      }
+      HIP_OK(launch_cone(a, s));
+      std::swap(cur, next);
     }
-    HIP_OK(launch_extract_box(out_dev ? out : design_out.as<double>(), cur, d.nx, d.ny, d.nz, dbox, s));
     HIP_OK(hipEventRecord(ev[1], s));
     if (!out_dev) HIP_OK(hipMemcpyAsync(out, design_out.p, (size_t)ND * 8, hipMemcpyDeviceToHost, s));
     HIP_OK(hipStreamSynchronize(s));
@@ -296,8 +322,11 @@ lbmx_status filter_design(lbmx_filter* h, const double* design, size_t nd, doubl
   return guarded([&] {
     lbmx::Filter& F = *h->f;
     F.check_sizes(nd, nf, physical != nullptr);
-    const double* x = F.run_design(design, dev, F.own);
-    if (physical)
+    // the only stage reads the design while it writes: a physical field that shares memory with
+    // the design is copied afterwards
+    const bool shared = dev && physical && F.stages.size() == 1 && physical < design + F.ND && design < physical + F.N;
+    const double* x = F.run_design(design, dev, dev && !shared ? physical : nullptr, F.own);
+    if (physical && (!dev || shared))
       HIP_OK(hipMemcpyAsync(physical, x, (size_t)F.N * 8, dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost,
                             F.own));
     HIP_OK(hipStreamSynchronize(F.own));
@@ -320,7 +349,7 @@ lbmx_status filter_design_to_solver(lbmx_filter* h, const double* design, size_t
     F.check_sizes(nd, 0, false);
     check_solver_grid(F, s);
     hipStream_t st = lbmx::solver_stream(s);
-    const double* x = F.run_design(design, dev, st);
+    const double* x = F.run_design(design, dev, nullptr, st);
     lbmx::solver_set_design_device(s, x);
     HIP_OK(hipStreamSynchronize(st));
     F.finish_design_timing();

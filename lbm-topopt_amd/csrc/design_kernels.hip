@@ -1,28 +1,22 @@
 // Design pipeline kernels: design-box mapping, cone density filter (forward and transposed),
 // tanh projection and its sensitivity scaling. All fields are FP64 in natural order
 // (z*ny + y)*nx + x on the full grid.
-//
-// The cone filter sums its taps in ascending (dz, dy, dx) order with separately rounded
-// multiplies and adds. That is the order in which a compressed-row MatMult visits the columns
-// of a row, and the order in which MatMultTranspose accumulates into an entry, so the results
-// equal a plain row loop (and a scatter-form transpose) bit for bit.
 #include <hip/hip_runtime.h>
 
+#include "design_cone.hpp"
 #include "lbmx_launch.h"
 
 namespace lbmx {
 
 namespace {
 
+constexpr int kMaxR = 16;
+
+// ---- cone of any radius ----
 constexpr int kConeTX = 64;   // outputs along x per workgroup (one wave wide)
 constexpr int kConeWY = 4;    // waves per workgroup, stacked along y
 constexpr int kConeKY = 4;    // outputs per thread along y (four named sums in k_cone)
 constexpr int kConeTY = kConeWY * kConeKY;  // outputs along y per workgroup
-constexpr int kMaxR = 16;
-
-__device__ inline bool in_box(int x, int y, int z, const int* b) {
-  return x >= b[0] && x <= b[1] && y >= b[2] && y <= b[3] && z >= b[4] && z <= b[5];
-}
 
 // LDS bytes of one workgroup: the input region of one plane and that plane's cone weights
 inline size_t cone_lds_bytes(int R) {
@@ -49,7 +43,6 @@ __global__ __launch_bounds__(256) void k_cone(ConeArgs a) {
   const int y0 = blockIdx.y * kConeTY;
   const int z = blockIdx.z;
   const int x = x0 + tx;
-  const size_t plane = (size_t)a.nx * a.ny;
 
   double acc[kConeKY];
   double own[kConeKY];  // transposed: this output's own input (identity rows outside the box)
@@ -60,25 +53,15 @@ __global__ __launch_bounds__(256) void k_cone(ConeArgs a) {
     acc[k] = 0.0;
     const bool valid = x < a.nx && y < a.ny;
     mine[k] = valid && in_box(x, y, z, a.box);
-    own[k] = valid ? a.in[(size_t)z * plane + (size_t)y * a.nx + x] : 0.0;
+    own[k] = valid && a.transposed ? cone_input(a, x, y, z) : 0.0;
   }
 
   for (int dz = -R; dz <= R; ++dz) {
     const int zz = z + dz;
     if (zz < 0 || zz >= a.nz) continue;  // uniform over the workgroup
     __syncthreads();
-    for (int idx = threadIdx.x; idx < W * H; idx += blockDim.x) {
-      const int lx = idx % W;
-      const int ly = idx / W;
-      const int gx = x0 - R + lx;
-      const int gy = y0 - R + ly;
-      double v = 0.0;
-      if (gx >= 0 && gx < a.nx && gy >= 0 && gy < a.ny) {
-        // transposed: only rows inside the box carry cone weights
-        if (!a.transposed || in_box(gx, gy, zz, a.box)) v = a.in[(size_t)zz * plane + (size_t)gy * a.nx + gx];
-      }
-      tile[ly * W + lx] = v;
-    }
+    for (int idx = threadIdx.x; idx < W * H; idx += blockDim.x)
+      tile[idx] = cone_tile_value(a, x0 - R + idx % W, y0 - R + idx / W, zz);
     const double* wz = a.wt + (size_t)(dz + R) * S * S;
     for (int idx = threadIdx.x; idx < S * S; idx += blockDim.x) wl[idx] = wz[idx];
     __syncthreads();
@@ -144,16 +127,16 @@ __global__ __launch_bounds__(256) void k_cone(ConeArgs a) {
     }
   }
 
-#pragma unroll
+  // (the sums move down one by one, so that the code after them exists once)
+#pragma unroll 1
   for (int k = 0; k < kConeKY; ++k) {
     const int y = y0 + ty + kConeWY * k;
-    if (x >= a.nx || y >= a.ny) continue;
-    const size_t i = (size_t)z * plane + (size_t)y * a.nx + x;
-    double v;
-    if (a.transposed) v = acc[k];
-    else if (!mine[k]) v = own[k];
-    else v = a.den ? acc[k] / a.den[i] : acc[k];
-    a.out[i] = v;
+    if (x < a.nx && y < a.ny) {
+      double v = 0.0, p = 0.0;
+      cone_finish(a, x, y, z, acc[0], a.transposed ? 1.0 : cone_second(a, x, y, z), v, p);
+      cone_store(a, x, y, z, v, p);
+    }
+    for (int i = 1; i < kConeKY; ++i) acc[i - 1] = acc[i];
   }
 }
 
@@ -173,73 +156,12 @@ struct Box6 {
   int b[6];
 };
 
-__global__ __launch_bounds__(256) void k_map_to_full(double* out, const double* design, const double* background,
-                                                      Grid3 g, Box6 bx) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  int x, y, z;
-  if (!g.locate(i, x, y, z)) return;
-  const int* b = bx.b;
-  if (in_box(x, y, z, b)) {
-    const int nxd = b[1] - b[0] + 1, nyd = b[3] - b[2] + 1;
-    out[i] = design[((size_t)(z - b[4]) * nyd + (y - b[2])) * nxd + (x - b[0])];
-  } else {
-    out[i] = background[i];
-  }
-}
-
-__global__ __launch_bounds__(256) void k_extract_box(double* design, const double* full, Grid3 g, Box6 bx) {
-  const int* b = bx.b;
-  const int nxd = b[1] - b[0] + 1, nyd = b[3] - b[2] + 1, nzd = b[5] - b[4] + 1;
-  const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= (long long)nxd * nyd * nzd) return;
-  const int xd = (int)(k % nxd);
-  const long long r = k / nxd;
-  const int yd = (int)(r % nyd);
-  const int zd = (int)(r / nyd);
-  design[k] = full[((size_t)(zd + b[4]) * g.ny + (yd + b[2])) * g.nx + (xd + b[0])];
-}
-
-// threshold of node i: the stage constant, or a per-node value with its own tanh terms
-__device__ inline void node_eta(const double* etaf, long long i, double beta, double& eta, double& tb,
-                                double& tsum) {
-#pragma clang fp contract(off)
-  if (etaf) {
-    eta = etaf[i];
-    tb = tanh(beta * eta);
-    tsum = tb + tanh(beta * (1.0 - eta));
-  }
-}
-
-__global__ __launch_bounds__(256) void k_project(double* out, const double* xin, Grid3 g, Box6 bx, double beta,
-                                                  double eta, double tb, double tsum, const double* etaf) {
-#pragma clang fp contract(off)
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  int x, y, z;
-  if (!g.locate(i, x, y, z)) return;
-  const double v = xin[i];
-  if (in_box(x, y, z, bx.b)) {
-    node_eta(etaf, i, beta, eta, tb, tsum);
-    out[i] = (tb + tanh(beta * (v - eta))) / tsum;
-  } else {
-    out[i] = v;
-  }
-}
-
 __global__ __launch_bounds__(256) void k_sens_scale(double* out, const double* sens, const double* xin,
-                                                     const double* den, Grid3 g, Box6 bx, int project, double beta,
-                                                     double eta, double tsum, const double* etaf) {
-#pragma clang fp contract(off)
+                                                     const double* den, Grid3 g, Box6 bx, ProjectArgs p) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   int x, y, z;
   if (!g.locate(i, x, y, z)) return;
-  double s = sens[i];
-  if (project && in_box(x, y, z, bx.b)) {
-    double tb = 0.0;
-    node_eta(etaf, i, beta, eta, tb, tsum);
-    const double t = tanh(beta * (xin[i] - eta));
-    s = s * (((1.0 - t * t) * beta) / tsum);
-  }
-  out[i] = s / den[i];
+  out[i] = scaled(p, in_box(x, y, z, bx.b), (size_t)i, sens[i], xin, den);
 }
 
 __global__ __launch_bounds__(256) void k_convert_f64_f32(float* out, const double* in, long long n) {
@@ -257,43 +179,26 @@ inline Box6 box6(const int b[6]) {
 
 }  // namespace
 
+// Radii up to these have a kernel of their own (2D: 2 x 2 outputs per lane, 3D: 2 x 4 x 4).
+// The unrolled taps fill about 30 KB of the 64 KB instruction cache at radius 12 in 2D and all
+// of it at radius 3 in 3D (32 x 123 taps per lane); larger radii take the kernel of any radius.
+constexpr int kConeFixed2D = 12;
+constexpr int kConeFixed3D = 3;
+
 hipError_t launch_cone(const ConeArgs& a, hipStream_t s) {
   if (a.R < 1 || a.R > kMaxR || a.nx < 1 || a.ny < 1 || a.nz < 1) return hipErrorInvalidValue;
+  if (a.nz == 1 && a.R <= kConeFixed2D) return a.R <= 8 ? launch_cone_2d_small(a, s) : launch_cone_2d_large(a, s);
+  if (a.nz > 1 && a.R <= kConeFixed3D) return launch_cone_3d_small(a, s);
   dim3 grid((a.nx + kConeTX - 1) / kConeTX, (a.ny + kConeTY - 1) / kConeTY, a.nz);
   hipLaunchKernelGGL(k_cone, grid, dim3(kConeTX * kConeWY), cone_lds_bytes(a.R), s, a);
   return hipGetLastError();
 }
 
-hipError_t launch_map_to_full(double* out, const double* design, const double* background, int nx, int ny, int nz,
-                              const int box[6], hipStream_t s) {
-  const long long n = (long long)nx * ny * nz;
-  hipLaunchKernelGGL(k_map_to_full, dim3(blocks_for(n)), dim3(256), 0, s, out, design, background,
-                     Grid3{nx, ny, nz}, box6(box));
-  return hipGetLastError();
-}
-
-hipError_t launch_extract_box(double* design, const double* full, int nx, int ny, int nz, const int box[6],
-                              hipStream_t s) {
-  const long long n = (long long)(box[1] - box[0] + 1) * (box[3] - box[2] + 1) * (box[5] - box[4] + 1);
-  hipLaunchKernelGGL(k_extract_box, dim3(blocks_for(n)), dim3(256), 0, s, design, full, Grid3{nx, ny, nz},
-                     box6(box));
-  return hipGetLastError();
-}
-
-hipError_t launch_project(double* out, const double* x, int nx, int ny, int nz, const int box[6], double beta,
-                          double eta, double tb, double tsum, const double* etaf, hipStream_t s) {
-  const long long n = (long long)nx * ny * nz;
-  hipLaunchKernelGGL(k_project, dim3(blocks_for(n)), dim3(256), 0, s, out, x, Grid3{nx, ny, nz}, box6(box), beta,
-                     eta, tb, tsum, etaf);
-  return hipGetLastError();
-}
-
 hipError_t launch_sens_scale(double* out, const double* sens, const double* x, const double* den, int nx, int ny,
-                             int nz, const int box[6], int project, double beta, double eta, double tsum,
-                             const double* etaf, hipStream_t s) {
+                             int nz, const int box[6], const ProjectArgs& p, hipStream_t s) {
   const long long n = (long long)nx * ny * nz;
   hipLaunchKernelGGL(k_sens_scale, dim3(blocks_for(n)), dim3(256), 0, s, out, sens, x, den, Grid3{nx, ny, nz},
-                     box6(box), project, beta, eta, tsum, etaf);
+                     box6(box), p);
   return hipGetLastError();
 }
 

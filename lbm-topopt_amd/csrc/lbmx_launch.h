@@ -29,32 +29,48 @@ hipError_t fill_zero(void* p, size_t bytes, hipStream_t s);
 hipError_t convert_f64_f32(float* out, const double* in, long long n, hipStream_t s);
 
 // Design pipeline kernels (natural-order FP64 fields on the full grid).
+// Projection of one stage: (tb + tanh(beta (x - eta))) / tsum with tb = tanh(beta eta) and
+// tsum = tb + tanh(beta (1 - eta)); with a per-node eta field (etaf != nullptr) eta, tb and
+// tsum are those of etaf[i].
+struct ProjectArgs {
+  int on;              // 0: the stage does not project
+  double beta, eta, tb, tsum;
+  const double* etaf;
+};
 struct ConeArgs {
-  const double* in;    // field to filter (forward) or s / (W 1) (transposed)
-  double* out;
+  // input: the full field `in`, or with design != nullptr the mapped field (inside dbox
+  // design[box-local i], elsewhere background[i])
+  const double* in;
+  const double* design;
+  const double* background;
+  double* out;         // full field: the filtered field (forward), W^T in (transposed)
   const double* den;   // forward: divide by den inside the box (nullptr: no division)
   const double* wt;    // weights [(dz+R)(2R+1) + dy+R][dx+R], (2R+1)^3 entries (2D: dz = 0 only)
+  const double* wd2;   // the same weights by squared offset: R - sqrt(d2), d2 = 0 .. R^2
   const int* rx;       // per (dz, dy): largest |dx| with dx^2+dy^2+dz^2 <= R^2, or -1
   int nx, ny, nz, R;
   int box[6];          // filter box, inclusive, clipped to the grid
+  int dbox[6];         // design box
   int transposed;      // 0: out = W in (rows in the box), 1: out = W^T in
+  // forward: projected field and a copy of the stage's output (either may be nullptr)
+  ProjectArgs proj;
+  double* proj_out;
+  double* copy_out;
+  // transposed, one of: design_out != nullptr: only the design box's entries, box-local;
+  // scale_den != nullptr: out = the result scaled for the stage before (its projection `proj`
+  // at its filtered field scale_x, divided by scale_den), see launch_sens_scale
+  double* design_out;
+  const double* scale_x;
+  const double* scale_den;
 };
 hipError_t launch_cone(const ConeArgs& a, hipStream_t s);
-// out[i] = inside design box ? design[box-local i] : background[i]
-hipError_t launch_map_to_full(double* out, const double* design, const double* background, int nx, int ny, int nz,
-                              const int box[6], hipStream_t s);
-// design[box-local i] = full[i] over the design box
-hipError_t launch_extract_box(double* design, const double* full, int nx, int ny, int nz, const int box[6],
-                              hipStream_t s);
-// out = inside box ? (tb + tanh(beta (x - eta))) / tsum : x, with tb = tanh(beta eta) and
-// tsum = tb + tanh(beta (1 - eta)); with a per-node eta field (etaf != nullptr) eta, tb and
-// tsum are those of etaf[i]
-hipError_t launch_project(double* out, const double* x, int nx, int ny, int nz, const int box[6], double beta,
-                          double eta, double tb, double tsum, const double* etaf, hipStream_t s);
+// (its kernels of one radius: 2D radii 1..8 and 9..12, 3D radii 1..3)
+hipError_t launch_cone_2d_small(const ConeArgs& a, hipStream_t s);
+hipError_t launch_cone_2d_large(const ConeArgs& a, hipStream_t s);
+hipError_t launch_cone_3d_small(const ConeArgs& a, hipStream_t s);
 // out = (inside box && project ? sens * (1 - tanh(beta (x - eta))^2) beta / tsum : sens) / den
 hipError_t launch_sens_scale(double* out, const double* sens, const double* x, const double* den, int nx, int ny,
-                             int nz, const int box[6], int project, double beta, double eta, double tsum,
-                             const double* etaf, hipStream_t s);
+                             int nz, const int box[6], const ProjectArgs& p, hipStream_t s);
 
 // Method of moving asymptotes: per-variable arrays of one optimiser (n variables, m <= 8
 // constraints; pij, qij, dgdx hold m rows of n) and the multipliers of a dual evaluation.
