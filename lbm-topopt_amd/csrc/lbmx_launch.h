@@ -72,30 +72,37 @@ hipError_t launch_cone_3d_small(const ConeArgs& a, hipStream_t s);
 hipError_t launch_sens_scale(double* out, const double* sens, const double* x, const double* den, int nx, int ny,
                              int nz, const int box[6], const ProjectArgs& p, hipStream_t s);
 
-// Method of moving asymptotes: per-variable arrays of one optimiser (n variables, m <= 8
-// constraints; pij, qij, dgdx hold m rows of n) and the multipliers of a dual evaluation.
+// Method of moving asymptotes: one update's per-variable inputs (n variables, m <= 8
+// constraints) and the dual iteration's state on the device.
 constexpr int kMmaMaxM = 8;
 struct MmaArgs {
   long long n;
   int m, k, con_mod, asym_type;
   double movlim, asyminit, asymdec, asyminc;
-  double* x;
+  const double* x;                 // the design the subproblem is built around
   const double* dfdx;
-  const double* dgdx;
-  const double* xo1;
-  const double* xo2;
-  double *lower, *upper, *L, *U, *alpha, *beta, *p0, *q0, *pij, *qij;
+  const double* dgdx[kMmaMaxM];    // constraint sensitivities, one row each
+  double *L, *U;                   // asymptotes (in: of the last update, out: of this one)
 };
-struct MmaLambda {
-  double lam[kMmaMaxM];
+struct MmaConsts {
+  double a[kMmaMaxM], c[kMmaMaxM], gx[kMmaMaxM];
+  double tol;                      // the iteration ends when epsi falls to this
+};
+struct MmaState {
+  double lam[kMmaMaxM], mu[kMmaMaxM], y[kMmaMaxM], b[kMmaMaxM];
+  double z, epsi, err;
+  int loop, newton_iters, done, started;
 };
 int mma_blocks(long long n);  // blocks of the reductions (partials per block)
-// subproblem at a.x; out[0..m) = sum_i pij / (U - x) + qij / (x - L)
-hipError_t launch_mma_gensub(const MmaArgs& a, double* part, double* out, hipStream_t s);
-// a.x = x(lam); out[0..m) = the same sums at x(lam); with hess, out[m + j*m + l] = the
-// Gauss-Newton part of the dual Hessian
-hipError_t launch_mma_dual(const MmaArgs& a, const MmaLambda& lm, bool hess, double* part, double* out,
-                           hipStream_t s);
+// The subproblem at a.x: asymptotes into a.L, a.U, the design into xkeep (which may be xo2), and
+// the state of a dual iteration that starts there.
+hipError_t launch_mma_gensub(const MmaArgs& a, const double* xo1, const double* xo2, double* xkeep, const MmaConsts& c,
+                             double* part, MmaState* state, hipStream_t s);
+// One Newton iteration of the dual (nothing once state->done is set): the sums at x(lam), the
+// residual they leave, and the next multipliers.
+hipError_t launch_mma_newton(const MmaArgs& a, const MmaConsts& c, double* part, MmaState* state, hipStream_t s);
+// xnew (and xnew2 unless nullptr) = x(lam)
+hipError_t launch_mma_primal(const MmaArgs& a, const MmaState* state, double* xnew, double* xnew2, hipStream_t s);
 // out[0] = max |xnew - xo1|
 hipError_t launch_mma_change(const double* xnew, const double* xo1, long long n, double* part, double* out,
                              hipStream_t s);
