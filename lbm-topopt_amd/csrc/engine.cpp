@@ -20,6 +20,8 @@
 #include "lbmx_common.h"
 #include "lbmx_device.hpp"
 #include "lbmx_launch.h"
+#include "lbmx_steps_shape.hpp"
+#include "sweep_plan.hpp"
 
 namespace lbmx {
 
@@ -122,6 +124,42 @@ static PassResult checkpointed_pass(SweepOps& ops, int nsteps, bool naive, std::
     if (!naive) sched->release();
   }
   return r;
+}
+
+// Lists the sweeps of a pass on numbered buffers instead of running them.
+struct RecordSweeps : SweepOps {
+  std::vector<SweepOp> ops;
+  std::unordered_map<const void*, int> id;
+  int of(const void* p) { return id.emplace(p, (int)id.size()).first->second; }
+  void init(void* dst) override { ops.push_back({SweepOp::kInit, -1, of(dst), 0, false}); }
+  void fwd(const void* src, void* dst, int t, bool with_obj) override {
+    const int a = of(src), b = of(dst);
+    ops.push_back({SweepOp::kFwd, a, b, t, with_obj});
+  }
+  void adj(const void* fsrc, const void*, void*, int t) override { ops.push_back({SweepOp::kAdj, of(fsrc), -1, t, false}); }
+};
+
+// A pass as launches: the checkpointed pass's sweeps, consecutive ones grouped. buffers[i] is
+// the buffer that the groups call i.
+struct SweepLaunches {
+  std::vector<SweepGroup> groups;
+  std::vector<void*> buffers;
+  PassResult result;
+};
+static SweepLaunches plan_launches(int nsteps, bool naive, std::vector<void*> slotbuf, void* work0, void* work1,
+                                   bool with_obj, int mode, int max_fwd, int max_adj) {
+  RecordSweeps rec;
+  std::vector<void*> all(slotbuf);
+  all.push_back(work0);
+  all.push_back(work1);
+  for (void* p : all) rec.of(p);
+  SweepLaunches l;
+  l.buffers = all;
+  char lam[2];
+  void *lin = &lam[0], *lout = &lam[1];
+  l.result = checkpointed_pass(rec, nsteps, naive, slotbuf, work0, work1, lin, lout, with_obj, mode);
+  l.groups = group_sweeps(rec.ops, (int)all.size(), max_fwd, max_adj);
+  return l;
 }
 
 struct Engine {
@@ -638,6 +676,75 @@ struct Engine {
     }
 #undef CALL
   }
+  // Several steps per launch: 2D lattices without Neumann pieces, whose transfers between nodes
+  // run between the sweeps. dir: 0 forward, 1 reverse.
+  bool steps_possible() const { return D == 2 && nside_count == 0; }
+  StepsShape steps_shape(int dir) const {
+    if (!steps_possible()) return {1, 1};
+    return lbmx::steps_shape(d, dir, (int)bcs.size(), N, [&](int H) {
+      return (long long)((d.nx + kTileX - 1) / kTileX) * ((d.ny + H - 1) / H);
+    });
+  }
+  void fill_steps(StepsCommon& c, int K, int H) const {
+    c.nx = d.nx;
+    c.ny = d.ny;
+    c.K = K;
+    c.H = H;
+    c.nbc = (int)bcs.size();
+    c.bcs = static_cast<const DevBC*>(bc_dev.p);
+    c.gamma = gamma_dev.p;
+    c.ls = ls;
+    c.m = params();
+    c.obj = obj;
+  }
+  // forward steps t, t + 1, .. from src in one launch; the state after the j-th goes to dst[j]
+  // (null: not kept; the last always is)
+  hipError_t run_fwd_steps(const void* src, void* const* dst, int t, int K, bool with_obj) {
+    if (K == 1) return run_fwd(fwd_args(src, dst[0], t, with_obj));
+    FwdSteps a{};
+    fill_steps(a.c, K, steps_shape(0).H);
+    a.c.obj.acc = (with_obj && obj_set && obj.nterm > 0) ? static_cast<double*>(acc_dev.p) : nullptr;
+    a.src = src;
+    a.t = t;
+    a.nblk_x = (d.nx + kTileX - 1) / kTileX;
+    a.nblocks = a.nblk_x * ((d.ny + a.c.H - 1) / a.c.H);
+    for (int j = 0; j < K; ++j) {
+      a.dst[j] = dst[j];
+      time_factors(t + j, a.tf + (size_t)j * kMaxBC);
+    }
+#define CALL(S) launch_fwd_steps_##S(d.collision, d.design, a, stream)
+    switch (d.lattice) {
+      case LBMX_D2Q9: LBMX_PREC_SWITCH(d2q9, CALL)
+      case LBMX_D2Q9_D2Q5: LBMX_PREC_SWITCH(thermal, CALL)
+      default: return hipErrorInvalidValue;
+    }
+#undef CALL
+  }
+  // reverse steps t, t - 1, .. in one launch; state[j] = p_{t-j-1}
+  hipError_t run_adj_steps(void* const* state, const void* lin, void* lout, int t, int K, const ObjArgs& oa) {
+    if (K == 1) return run_adj(adj_args(state[0], lin, lout, t, oa));
+    AdjSteps a{};
+    fill_steps(a.c, K, steps_shape(1).H);
+    a.c.obj = oa;
+    a.c.obj.acc = nullptr;
+    a.lam_in = lin;
+    a.lam_out = lout;
+    a.sens = static_cast<double*>(sens_dev.p);
+    a.ll = ll;
+    a.nblk_x = (d.nx + kTileX - 1) / kTileX;
+    a.nblocks = a.nblk_x * ((d.ny + a.c.H - 1) / a.c.H);
+    for (int j = 0; j < K; ++j) {
+      a.state[j] = state[j];
+      time_factors(t - j, a.tf + (size_t)j * kMaxBC);
+    }
+#define CALL(S) launch_adj_steps_##S(d.collision, d.design, a, stream)
+    switch (d.lattice) {
+      case LBMX_D2Q9: LBMX_PREC_SWITCH(d2q9, CALL)
+      case LBMX_D2Q9_D2Q5: LBMX_PREC_SWITCH(thermal, CALL)
+      default: return hipErrorInvalidValue;
+    }
+#undef CALL
+  }
   hipError_t run_init(const FwdArgs& a, const double* macros) {
 #define CALL(S) launch_init_##S(d.collision, d.design, a, macros, init_u, init_rho, init_T, stream)
     switch (d.lattice) {
@@ -766,11 +873,16 @@ struct Engine {
     bool with_obj = J && obj_set && obj.nterm > 0;
     if (with_obj) zero_acc();
     auto t0 = std::chrono::steady_clock::now();
-    for (int s = 0; s < nsteps; ++s) {
-      FwdArgs a = fwd_args(cur, prev, t + 1, with_obj);
-      HIP_OK(run_fwd(a));
+    // (the last step by itself: its input p_{t-1} stays available)
+    const int most = steps_shape(0).K;
+    for (int left = nsteps; left > 0;) {
+      const int k = left == 1 ? 1 : std::min(left - 1, most);
+      void* dst[kMaxSteps] = {};
+      dst[k - 1] = prev;
+      HIP_OK(run_fwd_steps(cur, dst, t + 1, k, with_obj));
       std::swap(cur, prev);
-      ++t;
+      t += k;
+      left -= k;
       state_kind = 0;
     }
     stats.fwd_sweeps += nsteps;
@@ -845,47 +957,50 @@ struct Engine {
     oa.acc = nullptr;
     if (!with_obj) oa.nterm = 0;
 
-    struct Ops : SweepOps {
-      Engine& e;
-      const ObjArgs& oa;
-      bool reverse_started = false;
-      std::chrono::steady_clock::time_point t_fwd_end;
-      Ops(Engine& en, const ObjArgs& o) : e(en), oa(o) {}
-      void init(void* dst) override {
-        FwdArgs a = e.fwd_args(nullptr, dst, 0, false);
-        HIP_OK(e.run_init(a, nullptr));
-        if (e.obj_set && e.obj.nterm > 0) e.zero_acc();
-      }
-      void fwd(const void* src, void* dst, int t, bool with) override {
-        FwdArgs a = e.fwd_args(src, dst, t, with);
-        HIP_OK(e.run_fwd(a));
-      }
-      void adj(const void* fsrc, const void* lin, void* lout, int t) override {
-        if (!reverse_started) {
-          reverse_started = true;
-          HIP_OK(hipStreamSynchronize(e.stream));  // end of the forward phase
-          t_fwd_end = std::chrono::steady_clock::now();
-          zero_async(e.lam_a.p, e.lam_bytes(), e.stream);
-          zero_async(e.sens_dev.p, (size_t)e.N * 8, e.stream);
-        }
-        AdjArgs a = e.adj_args(fsrc, lin, lout, t, oa);
-        HIP_OK(e.run_adj(a));
-      }
-    } ops(*this, oa);
-
+    const SweepLaunches plan =
+        plan_launches(nsteps, naive, slotbuf, pool[0]->p, pool[1]->p, with_obj, ckpt_mode, steps_shape(0).K,
+                      steps_shape(1).K);
+    const PassResult& pr = plan.result;
     auto tf0 = std::chrono::steady_clock::now();
+    std::chrono::steady_clock::time_point t_fwd_end;
     void* lin = lam_a.p;
     void* lout = lam_b.p;
-    PassResult pr =
-        checkpointed_pass(ops, nsteps, naive, slotbuf, pool[0]->p, pool[1]->p, lin, lout, with_obj, ckpt_mode);
+    bool reverse_started = false;
+    for (const SweepGroup& g : plan.groups) {
+      void* bufs[kMaxSteps] = {};
+      for (int j = 0; j < g.steps(); ++j) bufs[j] = g.buffers[j] < 0 ? nullptr : plan.buffers[g.buffers[j]];
+      switch (g.kind) {
+        case SweepOp::kInit: {
+          FwdArgs a = fwd_args(nullptr, bufs[0], 0, false);
+          HIP_OK(run_init(a, nullptr));
+          if (with_obj) zero_acc();
+          break;
+        }
+        case SweepOp::kFwd:
+          HIP_OK(run_fwd_steps(plan.buffers[g.src], bufs, g.t, g.steps(), g.with_obj));
+          break;
+        case SweepOp::kAdj: {
+          if (!reverse_started) {
+            reverse_started = true;
+            HIP_OK(hipStreamSynchronize(stream));  // end of the forward phase
+            t_fwd_end = std::chrono::steady_clock::now();
+            zero_async(lam_a.p, lam_bytes(), stream);
+            zero_async(sens_dev.p, (size_t)N * 8, stream);
+          }
+          HIP_OK(run_adj_steps(bufs, lin, lout, g.t, g.steps(), oa));
+          std::swap(lin, lout);
+          break;
+        }
+      }
+    }
     HIP_OK(hipStreamSynchronize(stream));
     auto tr1 = std::chrono::steady_clock::now();
     const double Jv = with_obj ? reduce_acc() : 0.0;
     stats.fwd_sweeps += nsteps + pr.recompute;
     stats.adj_sweeps += nsteps;
     stats.recompute_sweeps += pr.recompute;
-    stats.forward_phase_ms = std::chrono::duration<double, std::milli>(ops.t_fwd_end - tf0).count();
-    stats.reverse_phase_ms = std::chrono::duration<double, std::milli>(tr1 - ops.t_fwd_end).count();
+    stats.forward_phase_ms = std::chrono::duration<double, std::milli>(t_fwd_end - tf0).count();
+    stats.reverse_phase_ms = std::chrono::duration<double, std::milli>(tr1 - t_fwd_end).count();
     if (lin != lam_a.p) std::swap(lam_a.p, lam_b.p);  // final adjoint in lam_a
     sens_valid = adj_valid = true;
     adj_t = -1;
@@ -1090,14 +1205,16 @@ struct Batch {
   size_t state_total = 0, lam_total = 0;
   std::vector<BatchInst> inst;
   std::vector<int> blk_inst;
+  int steps_blocks[2] = {0, 0};  // workgroups of a launch of several steps (forward, reverse)
+  StepsShape steps[2] = {{1, 1}, {1, 1}};
   DeviceBuffer inst_dev, blk_dev, tfac_dev, lam_a, lam_b;
+  DeviceBuffer steps_blk_dev[2];
   std::vector<std::unique_ptr<DeviceBuffer>> pool;
   lbmx_stats stats{};
   std::vector<hipStream_t> member_streams;  // restored when the batch goes away
   bool use_graph = false;                   // replay the captured gradient pass
   hipGraphExec_t gexec = nullptr;
   std::vector<long long> gkey;              // what the captured graph was built for
-  long long graph_recompute = 0;
 
   explicit Batch(std::vector<Engine*> members) : m(std::move(members)) {
     if (m.empty()) throw Error{LBMX_ERR_ARG, "empty batch"};
@@ -1149,6 +1266,11 @@ struct Batch {
     auto ptr = [&](const void* p) { k.push_back((long long)(uintptr_t)p); };
     for (auto& p : pool) ptr(p->p);
     ptr(lam_a.p); ptr(lam_b.p); ptr(inst_dev.p); ptr(blk_dev.p); ptr(tfac_dev.p);
+    for (int dir = 0; dir < 2; ++dir) {
+      ptr(steps_blk_dev[dir].p);
+      k.push_back(steps[dir].K);
+      k.push_back(steps[dir].H);
+    }
     for (size_t i = 0; i < m.size(); ++i) {
       ptr(inst[i].obj.acc); ptr(inst[i].sens); ptr(inst[i].gamma); ptr(inst[i].bcs);
       k.push_back(inst[i].state_off);
@@ -1174,6 +1296,20 @@ struct Batch {
     nblocks = 0;
     tf_stride = 1;
     size_t st = 0, lt = 0;
+    long long nodes = 0;
+    for (Engine* e : m) nodes += e->N;
+    std::vector<int> steps_map[2];
+    size_t pieces = 0;
+    for (Engine* e : m) pieces = std::max(pieces, e->bcs.size());
+    auto tiles = [&](int H) {
+      long long n = 0;
+      for (Engine* e : m) n += (long long)((e->d.nx + kTileX - 1) / kTileX) * ((e->d.ny + H - 1) / H);
+      return n;
+    };
+    for (int dir = 0; dir < 2; ++dir) {
+      steps[dir] = m[0]->steps_possible() ? lbmx::steps_shape(m[0]->d, dir, (int)pieces, nodes, tiles) : StepsShape{1, 1};
+      steps_blocks[dir] = 0;
+    }
     for (size_t i = 0; i < m.size(); ++i) {
       Engine& e = *m[i];
       e.stream = stream;
@@ -1200,6 +1336,11 @@ struct Batch {
       st += align256(e.state_bytes());
       lt += align256(e.lam_bytes());
       for (int b = 0; b < g.nblocks; ++b) blk_inst.push_back((int)i);
+      for (int dir = 0; dir < 2; ++dir) {
+        I.steps_begin[dir] = steps_blocks[dir];
+        steps_blocks[dir] += g.nblk_x * ((e.d.ny + steps[dir].H - 1) / steps[dir].H);
+        steps_map[dir].resize((size_t)steps_blocks[dir], (int)i);
+      }
       nblocks += g.nblocks;
       tf_stride = std::max(tf_stride, I.nbc);
       inst.push_back(I);
@@ -1211,6 +1352,12 @@ struct Batch {
     HIP_OK(hipMemcpyAsync(inst_dev.p, inst.data(), inst.size() * sizeof(BatchInst), hipMemcpyHostToDevice, stream));
     blk_dev.ensure(blk_inst.size() * sizeof(int));
     HIP_OK(hipMemcpyAsync(blk_dev.p, blk_inst.data(), blk_inst.size() * sizeof(int), hipMemcpyHostToDevice, stream));
+    for (int dir = 0; dir < 2; ++dir) {
+      if (steps[dir].K == 1) continue;
+      steps_blk_dev[dir].ensure(steps_map[dir].size() * sizeof(int));
+      HIP_OK(hipMemcpyAsync(steps_blk_dev[dir].p, steps_map[dir].data(), steps_map[dir].size() * sizeof(int),
+                            hipMemcpyHostToDevice, stream));
+    }
     HIP_OK(hipStreamSynchronize(stream));
   }
 
@@ -1255,6 +1402,36 @@ struct Batch {
 #undef CALL
   }
 
+  // K = n forward steps t, t + 1, .. (states into bufs, null: not kept) or reverse steps t, t - 1,
+  // .. (on the states bufs) of every member in one launch
+  hipError_t launch_steps(int dir, const void* src, void* const* bufs, const void* lin, void* lout, int t, int n,
+                          bool with_obj) {
+    BatchSteps st{};
+    for (int j = 0; j < n; ++j) (dir ? const_cast<void*&>(st.state[j]) : st.dst[j]) = bufs[j];
+    if (!dir) st.state[0] = src;
+    st.lam_in = lin;
+    st.lam_out = lout;
+    st.inst = static_cast<const BatchInst*>(inst_dev.p);
+    st.blk_inst = static_cast<const int*>(steps_blk_dev[dir].p);
+    st.tf_stride = tf_stride;
+    const int per_step = (int)m.size() * tf_stride;
+    st.tfac = static_cast<const double*>(tfac_dev.p) + (size_t)t * per_step;
+    st.tf_step = dir ? -per_step : per_step;
+    st.K = n;
+    st.H = steps[dir].H;
+    st.nblocks = steps_blocks[dir];
+    st.t = t;
+    st.with_obj = with_obj ? 1 : 0;
+    const lbmx_desc& d = m[0]->d;
+#define CALL(S) launch_batch_steps_##S(d.collision, d.design, dir, st, stream)
+    switch (d.lattice) {
+      case LBMX_D2Q9: LBMX_BATCH_PREC(d2q9, CALL)
+      case LBMX_D2Q9_D2Q5: LBMX_BATCH_PREC(thermal, CALL)
+      default: return hipErrorInvalidValue;
+    }
+#undef CALL
+  }
+
   void init_all(void* dst, double rho0, const double* u0, double T0) {
     for (size_t i = 0; i < m.size(); ++i) {
       Engine& e = *m[i];
@@ -1294,50 +1471,58 @@ struct Batch {
     lam_b.ensure(lam_total);
     upload_tfac(nsteps);
 
-    struct Ops : SweepOps {
-      Batch& b;
-      double rho0, T0;
-      const double* u0;
-      bool capturing = false;
+    const SweepLaunches plan = plan_launches(nsteps, naive, slotbuf, pool[0]->p, pool[1]->p, true, ckpt_mode,
+                                             steps[0].K, steps[1].K);
+    const PassResult& pr = plan.result;
+    std::chrono::steady_clock::time_point t_fwd_end;
+    auto run_pass = [&](bool capturing) {
+      void* lin = lam_a.p;
+      void* lout = lam_b.p;
       bool reverse_started = false;
-      std::chrono::steady_clock::time_point t_fwd_end;
-      Ops(Batch& bb, double r, const double* u, double T) : b(bb), rho0(r), T0(T), u0(u) {}
-      void init(void* dst) override {
-        b.init_all(dst, rho0, u0, T0);
-        b.zero_accs();
-      }
-      void fwd(const void* src, void* dst, int t, bool with) override {
-        HIP_OK(b.launch(0, src, dst, nullptr, nullptr, t, with));
-      }
-      void adj(const void* fsrc, const void* lin, void* lout, int t) override {
-        if (!reverse_started) {
-          reverse_started = true;
-          if (!capturing) HIP_OK(hipStreamSynchronize(b.stream));  // end of the forward phase
-          t_fwd_end = std::chrono::steady_clock::now();
-          zero_async(b.lam_a.p, b.lam_total, b.stream);
-          for (auto& I : b.inst) zero_async(I.sens, (size_t)I.g.N * 8, b.stream);
+      for (const SweepGroup& g : plan.groups) {
+        const int n = g.steps();
+        void* bufs[kMaxSteps] = {};
+        for (int j = 0; j < n; ++j) bufs[j] = g.buffers[j] < 0 ? nullptr : plan.buffers[g.buffers[j]];
+        switch (g.kind) {
+          case SweepOp::kInit:
+            init_all(bufs[0], rho0, u0, T0);
+            zero_accs();
+            break;
+          case SweepOp::kFwd: {
+            const void* src = plan.buffers[g.src];
+            HIP_OK(n == 1 ? launch(0, src, bufs[0], nullptr, nullptr, g.t, g.with_obj)
+                          : launch_steps(0, src, bufs, nullptr, nullptr, g.t, n, g.with_obj));
+            break;
+          }
+          case SweepOp::kAdj:
+            if (!reverse_started) {
+              reverse_started = true;
+              if (!capturing) HIP_OK(hipStreamSynchronize(stream));  // end of the forward phase
+              t_fwd_end = std::chrono::steady_clock::now();
+              zero_async(lam_a.p, lam_total, stream);
+              for (auto& I : inst) zero_async(I.sens, (size_t)I.g.N * 8, stream);
+            }
+            HIP_OK(n == 1 ? launch(1, bufs[0], nullptr, lin, lout, g.t, true)
+                          : launch_steps(1, nullptr, bufs, lin, lout, g.t, n, true));
+            std::swap(lin, lout);
+            break;
         }
-        HIP_OK(b.launch(1, fsrc, nullptr, lin, lout, t, true));
       }
-    } ops(*this, rho0, u0, T0);
+    };
 
     auto tf0 = std::chrono::steady_clock::now();
-    void* lin = lam_a.p;
-    void* lout = lam_b.p;
-    PassResult pr;
     if (!use_graph) {
-      pr = checkpointed_pass(ops, nsteps, naive, slotbuf, pool[0]->p, pool[1]->p, lin, lout, true, ckpt_mode);
+      run_pass(false);
     } else {
       // the launch sequence of a pass is fixed by (steps, slots, tile height) and the buffer
       // addresses: capture it once, replay it on later calls
       std::vector<long long> key = graph_key(nsteps, slots, naive, rho0, u0, T0);
       if (!gexec || key != gkey) {
         drop_graph();
-        ops.capturing = true;
         HIP_OK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         hipGraph_t graph = nullptr;
         try {
-          pr = checkpointed_pass(ops, nsteps, naive, slotbuf, pool[0]->p, pool[1]->p, lin, lout, true, ckpt_mode);
+          run_pass(true);
         } catch (...) {
           (void)hipStreamEndCapture(stream, &graph);
           if (graph) (void)hipGraphDestroy(graph);
@@ -1351,12 +1536,10 @@ struct Batch {
           throw Error{LBMX_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(ie)};
         }
         gkey = key;
-        graph_recompute = pr.recompute;
       }
-      pr.recompute = graph_recompute;
       tf0 = std::chrono::steady_clock::now();
       HIP_OK(hipGraphLaunch(gexec, stream));
-      ops.t_fwd_end = tf0;  // phases are not separated inside a replay
+      t_fwd_end = tf0;  // phases are not separated inside a replay
     }
     HIP_OK(hipStreamSynchronize(stream));
     auto tr1 = std::chrono::steady_clock::now();
@@ -1373,8 +1556,8 @@ struct Batch {
     stats.fwd_sweeps += nsteps + pr.recompute;
     stats.adj_sweeps += nsteps;
     stats.recompute_sweeps += pr.recompute;
-    stats.forward_phase_ms = std::chrono::duration<double, std::milli>(ops.t_fwd_end - tf0).count();
-    stats.reverse_phase_ms = std::chrono::duration<double, std::milli>(tr1 - ops.t_fwd_end).count();
+    stats.forward_phase_ms = std::chrono::duration<double, std::milli>(t_fwd_end - tf0).count();
+    stats.reverse_phase_ms = std::chrono::duration<double, std::milli>(tr1 - t_fwd_end).count();
   }
 
   // Times nsweeps batched forward and adjoint sweeps for each tile shape (height 1, 2 or 4;
@@ -1759,6 +1942,33 @@ lbmx_status lbmx_checkpoint_simulate_mode(int nslots, int nsteps, int mode, long
                                 mode);
     *advances = r.recompute;
     *max_slots = r.max_slots;
+    // the same pass as launches of several steps, on labels
+    for (int k = 2; k <= lbmx::kMaxSteps; ++k) {
+      std::vector<void*> slots_again(slots);
+      for (int s = 0; s < slots; ++s) slots_again[s] = &storage[s];
+      const lbmx::SweepLaunches l =
+          lbmx::plan_launches(nsteps, false, slots_again, &storage[slots], &storage[slots + 1], false, mode, k, k);
+      std::vector<int> label(l.buffers.size(), -1);
+      int next = nsteps;
+      for (const lbmx::SweepGroup& g : l.groups) {
+        if (g.kind == lbmx::SweepOp::kFwd && label[g.src] != g.t - 1)
+          throw Error{LBMX_ERR_STATE, "grouped forward steps from " + std::to_string(g.t) + " read a wrong state"};
+        for (int j = 0; j < g.steps(); ++j) {
+          const int b = g.buffers[j];
+          if (g.kind == lbmx::SweepOp::kAdj) {
+            if (label[b] != g.t - j - 1 || g.t - j != next)
+              throw Error{LBMX_ERR_STATE, "grouped reverse steps: wrong state at step " + std::to_string(g.t - j)};
+            --next;
+          } else if (b >= 0) {
+            if (b == g.src) throw Error{LBMX_ERR_STATE, "a launch would write the state it reads"};
+            label[b] = g.kind == lbmx::SweepOp::kInit ? 0 : g.t + j;
+          } else if (j + 1 == g.steps()) {
+            throw Error{LBMX_ERR_STATE, "a launch without a result"};
+          }
+        }
+      }
+      if (next != 0) throw Error{LBMX_ERR_STATE, "grouped reverse steps are missing"};
+    }
   });
 }
 

@@ -1,0 +1,10 @@
+// Several steps per launch for D2Q9: incompressible BGK / MRT (forward + adjoint), cascaded and
+// standard BGK (forward); storage f64.
+#include "lbmx_steps.hpp"
+#include "lbmx_launch.h"
+#define LAT LatD2Q9
+#define PREC PrecF64
+#define SUFFIX d2q9_f64
+#define FWD_OPS X(C_BGK) X(C_MRT) X(C_CASC) X(C_BGK_STD)
+#define ADJ_OPS X(C_BGK) X(C_MRT)
+#include "lbmx_steps_dispatch.inc"

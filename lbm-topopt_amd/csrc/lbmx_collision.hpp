@@ -337,19 +337,31 @@ __device__ __forceinline__ void relax_even(Pairs<LatD3Q19, T>& p, Row&& row) {
 }  // namespace d3q19
 
 // ---- forward (pair space) ---------------------------------------------------------------
-template <class L, int COLL, int DES, class T>
+// WRITTEN: the two-product sums of the 2D BGK relaxation in a written-out fused form (with
+// Brinkman's term the other product is fused). Left to the compiler, which product it fuses
+// depends on what surrounds the inlined sum; the sweeps of one and of several steps have to
+// give the same bits.
+template <class L, int COLL, int DES, bool WRITTEN, class T>
 __device__ __forceinline__ void base_relax(Pairs<L, T>& p, T rho, const T (&v)[3], T omega, T alpha) {
   constexpr bool inc = CollTraits<COLL>::inc;
-  const T u2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+  constexpr bool written = WRITTEN && L::QF == 9;
+  T u2;
+  if constexpr (written) u2 = __builtin_elementwise_fma(v[0], v[0], v[1] * v[1]) + v[2] * v[2];
+  else u2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
   if constexpr (!CollTraits<COLL>::mrt) {
     // BGK: f' = f (1 - omega) + omega f_eq  (src/dynamics/incompressibleBGK2d.hh:38-47);
     // even/odd parts of f_eq: 2 w (rho + 4.5 cu^2 - 1.5 u^2), 2 w 3 cu (incompressible)
     const T one_m = T(1) - omega;
     const T kap_a = (T(1) - T(0.5) * omega) * alpha;
     const T rs = inc ? T(1) : rho;  // standard: f_eq = w rho (1 + ...)
+    auto relaxed = [&](T f, T eq) {
+      if constexpr (written && DES == D_BRINK) return __builtin_elementwise_fma(f, one_m, omega * eq);
+      else if constexpr (written) return __builtin_elementwise_fma(omega, eq, f * one_m);
+      else return f * one_m + omega * eq;
+    };
     {
       T feq0 = inc ? T(L::w[0]) * (rho - T(1.5) * u2) : T(L::w[0]) * rho * (T(1) - T(1.5) * u2);
-      T out = p.f0 * one_m + omega * feq0;
+      T out = relaxed(p.f0, feq0);
       if constexpr (DES == D_BRINK) out += kap_a * T(L::w[0]) * T(3) * u2;
       p.f0 = out;
     }
@@ -359,8 +371,7 @@ __device__ __forceinline__ void base_relax(Pairs<L, T>& p, T rho, const T (&v)[3
       const T w2 = T(2.0 * L::w[d]);
       T ev = inc ? w2 * (rho + T(4.5) * cu * cu - T(1.5) * u2) : w2 * rho * (T(1) + T(4.5) * cu * cu - T(1.5) * u2);
       T od = w2 * rs * T(3) * cu;
-      T s = p.s[d] * one_m + omega * ev;
-      T a = p.a[d] * one_m + omega * od;
+      T s = relaxed(p.s[d], ev), a = relaxed(p.a[d], od);
       if constexpr (DES == D_BRINK) {
         s -= kap_a * w2 * (T(9) * cu * cu - T(3) * u2);
         a -= kap_a * w2 * T(3) * cu;
@@ -390,7 +401,9 @@ __device__ __forceinline__ void base_relax(Pairs<L, T>& p, T rho, const T (&v)[3
         constexpr bool own_rate = LBMX_BAS.rate[k] == 1;
         T sk = own_rate ? omega : s_k;
         T val = sk * (mk - meq_row<L, k>(rho, vm, inv_rho_s));
-        if constexpr (DES == D_BRINK && row_has_src<L, k>())
+        if constexpr (written && DES == D_BRINK && row_has_src<L, k>())
+          val = __builtin_elementwise_fma((T(1) - T(0.5) * sk) * alpha, src_row<L, k>(v, u2), val);
+        else if constexpr (DES == D_BRINK && row_has_src<L, k>())
           val += (T(1) - T(0.5) * sk) * alpha * src_row<L, k>(v, u2);
         pair_row_update<L, k>(p, val * inv_n2);
       } else if constexpr (DES == D_BRINK && row_has_src<L, k>()) {
@@ -699,7 +712,7 @@ __device__ __forceinline__ void darcy_force(T (&f)[9], T rho, const T (&j)[3], T
 }
 
 // Moment-space operators (BGK, MRT): node collision in place; rho, j are the pre-collision macros.
-template <class L, int COLL, int DES, class T, bool TWICE = false>
+template <class L, int COLL, int DES, class T, bool TWICE, bool WRITTEN>
 __device__ __forceinline__ void collide_moment(T (&f)[L::Q], T gamma, const ModelParams& mp, T& rho, T (&j)[3]) {
   static_assert(!(TWICE && DES == D_DARCY), "the Darcy force acts on the populations themselves");
   Pairs<L, T> p;
@@ -714,7 +727,7 @@ __device__ __forceinline__ void collide_moment(T (&f)[L::Q], T gamma, const Mode
   if constexpr (DES == D_BRINK) alpha = mpar<T>(mp.alpha_max, mp.alpha_max_f) * bp_val<T>(mpar<T>(mp.interp_q, mp.interp_q_f), gamma);
   eq_velocity<L, COLL, DES>(rho, j, alpha, v, beta);
   if constexpr (grouped) relax_d3q19<COLL, DES>(p, rho, v, omega, alpha);
-  else base_relax<L, COLL, DES>(p, rho, v, omega, alpha);
+  else base_relax<L, COLL, DES, WRITTEN>(p, rho, v, omega, alpha);
   if constexpr (DES == D_PBB) {
     // PartialBouncebackCollision (src/dynamics/partialBouncebackCollision.hh:53-65): the
     // pair blend keeps f_d + f_d' and scales f_d - f_d' by 1 - 2 imult
@@ -751,7 +764,9 @@ __device__ __forceinline__ void reverse_moment(const T (&f)[L::Q], T gamma, cons
   T alpha = 0, beta, v[3];
   if constexpr (DES == D_BRINK) alpha = mpar<T>(mp.alpha_max, mp.alpha_max_f) * bp_val<T>(mpar<T>(mp.interp_q, mp.interp_q_f), gamma);
   eq_velocity<L, COLL, DES>(rho, j, alpha, v, beta);
-  const T u2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+  T u2;
+  if constexpr (L::QF == 9 && !CollTraits<COLL>::mrt) u2 = __builtin_elementwise_fma(v[0], v[0], v[1] * v[1]) + v[2] * v[2];
+  else u2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
   T gbar = 0;
   T lamT[L::QT > 0 ? 5 : 1];
   if constexpr (L::QT > 0) {
@@ -766,7 +781,10 @@ __device__ __forceinline__ void reverse_moment(const T (&f)[L::Q], T gamma, cons
     if constexpr (!CollTraits<COLL>::mrt) {
       static_for<1, H + 1>([&](auto dc) {
         constexpr int d = decltype(dc)::value;
-        gd[d] = pf.a[d] * (T(1) - omega) + omega * T(6.0 * L::w[d]) * cdot<L, d>(v);
+        // (2D: the fused form written out, see base_relax)
+        if constexpr (L::QF == 9)
+          gd[d] = __builtin_elementwise_fma(pf.a[d], T(1) - omega, omega * T(6.0 * L::w[d]) * cdot<L, d>(v));
+        else gd[d] = pf.a[d] * (T(1) - omega) + omega * T(6.0 * L::w[d]) * cdot<L, d>(v);
       });
     } else {
       Pairs<L, T> g;
@@ -796,36 +814,55 @@ __device__ __forceinline__ void reverse_moment(const T (&f)[L::Q], T gamma, cons
 
   T rho_bar = 0, vb[3] = {0, 0, 0}, alpha_bar = 0;
   if constexpr (!CollTraits<COLL>::mrt) {
+    // 2D: sums of two products in a written-out fused form, see base_relax
+    constexpr bool written = L::QF == 9;
     const T kap = T(1) - T(0.5) * omega;
     T S0 = T(L::w[0]) * pl.f0;
     T ce[3] = {0, 0, 0};  // sum_d w_d (3 c_d la_d + 9 cu_d c_d ls_d)
     T cs[3] = {0, 0, 0};  // sum_d w_d (3 c_d la_d + 18 cu_d c_d ls_d) (source)
-    T asum = 0;           // sum_d w_d (3 cu_d la_d + (9 cu_d^2 - 3 u2) ls_d) + w0 l0 (-3 u2)
+    T& asum = alpha_bar;  // sum_d w_d (3 cu_d la_d + (9 cu_d^2 - 3 u2) ls_d) + w0 l0 (-3 u2)
     if constexpr (DES == D_BRINK) asum = T(L::w[0]) * pl.f0 * (-T(3) * u2);
     static_for<1, H + 1>([&](auto dc) {
       constexpr int d = decltype(dc)::value;
       const T cu = cdot<L, d>(v);
       const T wd = T(L::w[d]);
-      S0 += wd * pl.s[d];
-      const T t1 = wd * (T(3) * pl.a[d] + T(9) * cu * pl.s[d]);
+      if constexpr (written && d == 1 && DES != D_BRINK) S0 = __builtin_elementwise_fma(T(L::w[0]), pl.f0, wd * pl.s[d]);
+      else if constexpr (written) S0 = __builtin_elementwise_fma(wd, pl.s[d], S0);
+      else S0 += wd * pl.s[d];
+      T t1;
+      if constexpr (written && DES == D_NONE) t1 = wd * __builtin_elementwise_fma(T(3), pl.a[d], T(9) * cu * pl.s[d]);
+      else if constexpr (written) t1 = wd * __builtin_elementwise_fma(T(9) * cu, pl.s[d], T(3) * pl.a[d]);
+      else t1 = wd * (T(3) * pl.a[d] + T(9) * cu * pl.s[d]);
       if constexpr (L::ex[d] != 0) ce[0] += T(L::ex[d]) * t1;
       if constexpr (L::ey[d] != 0) ce[1] += T(L::ey[d]) * t1;
       if constexpr (L::ez[d] != 0) ce[2] += T(L::ez[d]) * t1;
       if constexpr (DES == D_BRINK) {
-        const T t2 = wd * (T(3) * pl.a[d] + T(18) * cu * pl.s[d]);
+        T t2;
+        if constexpr (written) t2 = wd * __builtin_elementwise_fma(T(18) * cu, pl.s[d], T(3) * pl.a[d]);
+        else t2 = wd * (T(3) * pl.a[d] + T(18) * cu * pl.s[d]);
         if constexpr (L::ex[d] != 0) cs[0] += T(L::ex[d]) * t2;
         if constexpr (L::ey[d] != 0) cs[1] += T(L::ey[d]) * t2;
         if constexpr (L::ez[d] != 0) cs[2] += T(L::ez[d]) * t2;
-        asum += wd * (T(3) * cu * pl.a[d] + (T(9) * cu * cu - T(3) * u2) * pl.s[d]);
+        if constexpr (written)
+          asum = __builtin_elementwise_fma(
+              wd,
+              __builtin_elementwise_fma(T(3) * cu, pl.a[d],
+                                        __builtin_elementwise_fma(T(9) * cu, cu, -(T(3) * u2)) * pl.s[d]),
+              asum);
+        else asum += wd * (T(3) * cu * pl.a[d] + (T(9) * cu * cu - T(3) * u2) * pl.s[d]);
       }
     });
     rho_bar = omega * S0;
     static_for<0, 3>([&](auto ac) {
       constexpr int a = decltype(ac)::value;
-      vb[a] = omega * (ce[a] - T(3) * v[a] * S0);
-      if constexpr (DES == D_BRINK) vb[a] -= alpha * kap * (cs[a] - T(6) * v[a] * S0);
+      if constexpr (written && DES == D_BRINK) {
+        vb[a] = __builtin_elementwise_fma(omega, ce[a] - T(3) * v[a] * S0, -(alpha * kap * (cs[a] - T(6) * v[a] * S0)));
+      } else {
+        vb[a] = omega * (ce[a] - T(3) * v[a] * S0);
+        if constexpr (DES == D_BRINK) vb[a] -= alpha * kap * (cs[a] - T(6) * v[a] * S0);
+      }
     });
-    if constexpr (DES == D_BRINK) alpha_bar = -kap * asum;
+    if constexpr (DES == D_BRINK && L::QF != 9) alpha_bar = -kap * asum;
     const T one_m = T(1) - omega;
     pl.f0 *= one_m;
     static_for<1, H + 1>([&](auto dc) {
@@ -891,7 +928,17 @@ __device__ __forceinline__ void reverse_moment(const T (&f)[L::Q], T gamma, cons
   T jb[3] = {beta * vb[0] + srcB[0], beta * vb[1] + srcB[1], beta * vb[2] + srcB[2]};
   rho_bar += srcA;
   if constexpr (DES == D_BRINK) {
-    alpha_bar -= T(0.5) * beta * beta * (vb[0] * j[0] + vb[1] * j[1] + vb[2] * j[2]);
+    T vj;
+    if constexpr (!CollTraits<COLL>::mrt && L::Q == 9)
+      vj = __builtin_elementwise_fma(vb[0], j[0], vb[1] * j[1]) + vb[2] * j[2];
+    else if constexpr (!CollTraits<COLL>::mrt && L::QF == 9)
+      vj = __builtin_elementwise_fma(vb[1], j[1], vb[0] * j[0]) + vb[2] * j[2];
+    else vj = vb[0] * j[0] + vb[1] * j[1] + vb[2] * j[2];
+    const T half_b2 = T(0.5) * beta * beta * vj;
+    // 2D BGK (alpha_bar holds the sum before its factor): the fused form written out, see base_relax
+    if constexpr (!CollTraits<COLL>::mrt && L::QF == 9)
+      alpha_bar = __builtin_elementwise_fma(alpha_bar, T(0.5) * omega - T(1), -half_b2);
+    else alpha_bar -= half_b2;
     gbar += alpha_bar * mpar<T>(mp.alpha_max, mp.alpha_max_f) * bp_der<T>(mpar<T>(mp.interp_q, mp.interp_q_f), gamma);
   }
 
@@ -963,12 +1010,12 @@ template <int COLL, int DES>
 inline constexpr bool kCollideTwice = COLL != C_CASC && DES != D_DARCY;
 
 // Node collision in place; rho, j receive the pre-collision macros. TWICE (only where
-// kCollideTwice): f_q comes back doubled for q = 1 .. QF - 1.
-template <class L, int COLL, int DES, class T, bool TWICE = false>
+// kCollideTwice): f_q comes back doubled for q = 1 .. QF - 1. WRITTEN: see base_relax.
+template <class L, int COLL, int DES, class T, bool TWICE = false, bool WRITTEN = true>
 __device__ __forceinline__ void collide(T (&f)[L::Q], T gamma, const ModelParams& mp, T& rho, T (&j)[3]) {
   static_assert(!TWICE || kCollideTwice<COLL, DES>, "operator without a final halving");
   if constexpr (COLL == C_CASC) collide_cascaded<L, DES>(f, gamma, mp, rho, j);
-  else collide_moment<L, COLL, DES, T, TWICE>(f, gamma, mp, rho, j);
+  else collide_moment<L, COLL, DES, T, TWICE, WRITTEN>(f, gamma, mp, rho, j);
 }
 
 // lam <- (dC/df)^T lam + functional source; dgam += (dC/dgamma)^T lam.

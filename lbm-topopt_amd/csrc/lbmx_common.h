@@ -137,6 +137,38 @@ struct AdjArgs {
   ObjArgs obj;
 };
 
+// K forward steps of a 2D lattice in one launch (tiles of 64 x H nodes): dst = state after step
+// t + K - 1 from src = the state before step t. g's tiles are those of this launch.
+constexpr int kMaxSteps = 4;
+// What both directions need of a lattice and a launch.
+struct StepsCommon {
+  int nx, ny, K, H, nbc;
+  const DevBC* bcs;
+  const void* gamma;
+  Layout ls;
+  ModelParams m;
+  ObjArgs obj;
+};
+struct FwdSteps {
+  StepsCommon c;
+  const void* src;
+  void* dst[kMaxSteps];  // where the state after each step goes (null: not kept; the last is)
+  int t;              // time of the first new state
+  int nblk_x, nblocks;
+  double tf[kMaxSteps * kMaxBC];  // time factor of piece b at step t + j: [j * kMaxBC + b]
+};
+// K reverse steps t, t - 1, .. in one launch; state[j] = p_{t-j-1}
+struct AdjSteps {
+  StepsCommon c;
+  const void* state[kMaxSteps];
+  const void* lam_in;
+  void* lam_out;
+  double* sens;
+  Layout ll;
+  int nblk_x, nblocks;
+  double tf[kMaxSteps * kMaxBC];  // time factor of piece b at step t - j
+};
+
 // One instance of a batch: its static description for the batched sweeps.
 struct BatchInst {
   Geometry g;             // grid and tiles (for the batch's tile height)
@@ -149,6 +181,7 @@ struct BatchInst {
   const unsigned long long* bcrows;  // pieces meeting each 64-node row segment (bc_row_index)
   int nbc;
   int blk_begin;          // first global workgroup of this instance
+  int steps_begin[2];     // the same in launches of several steps (forward, reverse)
   long long state_off;    // byte offset of the instance in the batch state buffers
   long long lam_off;      // byte offset in the batch adjoint buffers
 };
@@ -166,6 +199,24 @@ struct BatchStep {
   int nblocks;            // total workgroups
   int t;                  // time of the new state (forward) / reverse step (adjoint)
   int with_obj;           // forward: accumulate the functional; adjoint: add its source
+};
+
+// Several steps of a batch in one launch (2D lattices): forward steps t .. t + K - 1 from src,
+// or reverse steps t .. t - K + 1 on the states src (state[j] = p_{t-j-1}).
+struct BatchSteps {
+  const void* state[kMaxSteps];  // forward: state[0] is the source
+  void* dst[kMaxSteps];   // forward: where each state goes (null: not kept)
+  const void* lam_in;
+  void* lam_out;
+  const BatchInst* inst;
+  const int* blk_inst;    // instance of each (XCD-remapped) workgroup of these tiles
+  const double* tfac;     // time factors of step t: [instance][tf_stride]
+  int tf_stride;          // most pieces of any member
+  int tf_step;            // doubles from one step's factors to the next step's (reverse: negative)
+  int K, H;
+  int nblocks;
+  int t;
+  int with_obj;
 };
 
 // Q directions c_q = (ex[q], ey[q], ez[q]) of the field's lattice

@@ -759,7 +759,7 @@ __global__ __launch_bounds__(kTileX* kTileY) void k_init(FwdArgs a, const double
     const T gam = T(static_cast<const typename P::G*>(a.gamma)[n]);
     T rho, j[3];
     constexpr bool tw = kStoreTwice<P, COLL, DES>;
-    collide<L, COLL, DES, T, tw>(f, gam, a.m, rho, j);
+    collide<L, COLL, DES, T, tw, false>(f, gam, a.m, rho, j);
     store_node<L, P, tw>(a.dst, a.ls, layout_off(a.ls, x, y, z), f, on_boundary<L>(x, y, z, nx, ny, nz), x, y, z, nx,
                      ny, nz, 0);
   }

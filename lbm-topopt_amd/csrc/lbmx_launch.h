@@ -22,6 +22,15 @@ LBMX_DECLARE_LATTICE(thermal)
 #undef LBMX_DECLARE_LATTICE
 #undef LBMX_DECLARE_LAUNCHERS
 
+// Several steps per launch (2D lattices): single lattices and batches (kind 0 forward, 1 reverse).
+#define LBMX_DECLARE_STEPS(SUFFIX)                                                              \
+  hipError_t launch_fwd_steps_##SUFFIX(int coll, int des, const FwdSteps& a, hipStream_t s);    \
+  hipError_t launch_adj_steps_##SUFFIX(int coll, int des, const AdjSteps& a, hipStream_t s);    \
+  hipError_t launch_batch_steps_##SUFFIX(int coll, int des, int kind, const BatchSteps& st, hipStream_t s);
+LBMX_DECLARE_STEPS(d2q9_f64) LBMX_DECLARE_STEPS(d2q9_f32) LBMX_DECLARE_STEPS(d2q9_f16) LBMX_DECLARE_STEPS(d2q9_bf16)
+LBMX_DECLARE_STEPS(thermal_f64) LBMX_DECLARE_STEPS(thermal_f32) LBMX_DECLARE_STEPS(thermal_f16) LBMX_DECLARE_STEPS(thermal_bf16)
+#undef LBMX_DECLARE_STEPS
+
 // Zero fill of a device range (bytes a multiple of 4) by a kernel.
 hipError_t fill_zero(void* p, size_t bytes, hipStream_t s);
 
