@@ -14,7 +14,6 @@
 #include <unordered_map>
 #include <vector>
 
-#include "checkpoint.hpp"
 #include "host_common.hpp"
 #include "lbmx.h"
 #include "lbmx_common.h"
@@ -37,130 +36,6 @@ static size_t prec_gamma_bytes(int prec) { return prec == LBMX_FP64 ? 8 : 4; }
 
 // zero fill by a kernel (also valid inside a captured graph)
 static void zero_async(void* p, size_t bytes, hipStream_t s) { HIP_OK(fill_zero(p, bytes, s)); }
-
-// The sweeps of one design-gradient pass, over opaque state buffers (a single lattice, a batch
-// of lattices in lockstep, or labelled host buffers that check the schedule).
-struct SweepOps {
-  virtual ~SweepOps() = default;
-  virtual void init(void* dst) = 0;                                              // p_0
-  virtual void fwd(const void* src, void* dst, int t, bool with_obj) = 0;       // p_t from p_{t-1}
-  virtual void adj(const void* fsrc, const void* lin, void* lout, int t) = 0;  // nu_{t-1} from nu_t
-};
-
-struct PassResult {
-  long long recompute = 0;  // forward sweeps re-run in the reverse phase
-  int max_slots = 0;        // slots in use at most
-};
-
-// Forward phase storing checkpoints in `slotbuf` (Wang dynamic checkpointing, or every state
-// when naive), then the reverse phase: the adjoint sweep at step t needs p_{t-1}, restored from
-// the nearest checkpoint and re-advanced (LBDynamicCheckpointing, src/topOpt/LBCheckpointing.cc:42-48;
-// WangCheckpointing::getForwardSolution, src/topOpt/WangCheckpointing.cc:36-126). Storing a
-// checkpoint swaps buffer handles (no copy). On return, lin holds the final adjoint nu_0.
-static PassResult checkpointed_pass(SweepOps& ops, int nsteps, bool naive, std::vector<void*>& slotbuf,
-                                    void* work0, void* work1, void*& lin, void*& lout, bool with_obj,
-                                    int mode = LBMX_CHECKPOINT_DYNAMIC) {
-  const int slots = (int)slotbuf.size();
-  void* work[2] = {work0, work1};
-  auto other_work = [&](const void* src) -> void*& { return src == work[0] ? work[1] : work[0]; };
-  std::unique_ptr<WangSchedule> sched;
-  if (!naive) {
-    sched.reset(new WangSchedule(slots));
-    if (mode == LBMX_CHECKPOINT_STATIC) sched->plan_static(nsteps - 1);
-    if (mode == LBMX_CHECKPOINT_BINOMIAL) sched->plan_binomial(nsteps);
-  }
-  PassResult r;
-  auto used = [&]() { r.max_slots = std::max(r.max_slots, naive ? slots : slots - sched->free_slots()); };
-  ops.init(work[0]);
-  auto store = [&](int step, void*& holder) -> void* {
-    int s = naive ? step : sched->make_checkpoint(step);
-    if (s < 0) return holder;       // a static schedule does not keep this step
-    std::swap(slotbuf[s], holder);  // the slot now owns the state; holder gets a spare buffer
-    return slotbuf[s];
-  };
-  void* src = store(0, work[0]);
-  used();
-  const void* last_input = nullptr;  // p_{nsteps-1}, the input of the last forward sweep
-  for (int k = 1; k <= nsteps; ++k) {
-    void*& dst = other_work(src);
-    if (k == nsteps) last_input = src;
-    ops.fwd(src, dst, k, with_obj);
-    if (k < nsteps) src = store(k, dst);
-    else src = dst;
-    used();
-  }
-  for (int step = nsteps; step >= 1; --step) {
-    const int index = step - 1;
-    const void* fsrc = nullptr;
-    if (naive) {
-      fsrc = slotbuf[index];
-    } else {
-      WangSchedule::Plan plan = sched->get_forward_solution(index);
-      if (plan.stored()) {
-        // a binomial plan may hand the first reverse step the forward pass's last input
-        fsrc = plan.from_slot >= 0 ? slotbuf[plan.from_slot] : last_input;
-      } else {
-        const void* s2 = slotbuf[plan.from_slot];
-        size_t next = 0;
-        for (int c = plan.from_step + 1; c <= plan.index; ++c) {
-          void*& dst = other_work(s2);
-          ops.fwd(s2, dst, c, false);
-          ++r.recompute;
-          if (next < plan.stores.size() && plan.stores[next].first == c) {
-            int s = plan.stores[next].second;
-            std::swap(slotbuf[s], dst);
-            s2 = slotbuf[s];
-            ++next;
-          } else {
-            s2 = dst;
-          }
-        }
-        fsrc = s2;
-      }
-      used();
-    }
-    ops.adj(fsrc, lin, lout, step);
-    std::swap(lin, lout);
-    if (!naive) sched->release();
-  }
-  return r;
-}
-
-// Lists the sweeps of a pass on numbered buffers instead of running them.
-struct RecordSweeps : SweepOps {
-  std::vector<SweepOp> ops;
-  std::unordered_map<const void*, int> id;
-  int of(const void* p) { return id.emplace(p, (int)id.size()).first->second; }
-  void init(void* dst) override { ops.push_back({SweepOp::kInit, -1, of(dst), 0, false}); }
-  void fwd(const void* src, void* dst, int t, bool with_obj) override {
-    const int a = of(src), b = of(dst);
-    ops.push_back({SweepOp::kFwd, a, b, t, with_obj});
-  }
-  void adj(const void* fsrc, const void*, void*, int t) override { ops.push_back({SweepOp::kAdj, of(fsrc), -1, t, false}); }
-};
-
-// A pass as launches: the checkpointed pass's sweeps, consecutive ones grouped. buffers[i] is
-// the buffer that the groups call i.
-struct SweepLaunches {
-  std::vector<SweepGroup> groups;
-  std::vector<void*> buffers;
-  PassResult result;
-};
-static SweepLaunches plan_launches(int nsteps, bool naive, std::vector<void*> slotbuf, void* work0, void* work1,
-                                   bool with_obj, int mode, int max_fwd, int max_adj) {
-  RecordSweeps rec;
-  std::vector<void*> all(slotbuf);
-  all.push_back(work0);
-  all.push_back(work1);
-  for (void* p : all) rec.of(p);
-  SweepLaunches l;
-  l.buffers = all;
-  char lam[2];
-  void *lin = &lam[0], *lout = &lam[1];
-  l.result = checkpointed_pass(rec, nsteps, naive, slotbuf, work0, work1, lin, lout, with_obj, mode);
-  l.groups = group_sweeps(rec.ops, (int)all.size(), max_fwd, max_adj);
-  return l;
-}
 
 struct Engine {
   lbmx_desc d{};
@@ -1942,33 +1817,6 @@ lbmx_status lbmx_checkpoint_simulate_mode(int nslots, int nsteps, int mode, long
                                 mode);
     *advances = r.recompute;
     *max_slots = r.max_slots;
-    // the same pass as launches of several steps, on labels
-    for (int k = 2; k <= lbmx::kMaxSteps; ++k) {
-      std::vector<void*> slots_again(slots);
-      for (int s = 0; s < slots; ++s) slots_again[s] = &storage[s];
-      const lbmx::SweepLaunches l =
-          lbmx::plan_launches(nsteps, false, slots_again, &storage[slots], &storage[slots + 1], false, mode, k, k);
-      std::vector<int> label(l.buffers.size(), -1);
-      int next = nsteps;
-      for (const lbmx::SweepGroup& g : l.groups) {
-        if (g.kind == lbmx::SweepOp::kFwd && label[g.src] != g.t - 1)
-          throw Error{LBMX_ERR_STATE, "grouped forward steps from " + std::to_string(g.t) + " read a wrong state"};
-        for (int j = 0; j < g.steps(); ++j) {
-          const int b = g.buffers[j];
-          if (g.kind == lbmx::SweepOp::kAdj) {
-            if (label[b] != g.t - j - 1 || g.t - j != next)
-              throw Error{LBMX_ERR_STATE, "grouped reverse steps: wrong state at step " + std::to_string(g.t - j)};
-            --next;
-          } else if (b >= 0) {
-            if (b == g.src) throw Error{LBMX_ERR_STATE, "a launch would write the state it reads"};
-            label[b] = g.kind == lbmx::SweepOp::kInit ? 0 : g.t + j;
-          } else if (j + 1 == g.steps()) {
-            throw Error{LBMX_ERR_STATE, "a launch without a result"};
-          }
-        }
-      }
-      if (next != 0) throw Error{LBMX_ERR_STATE, "grouped reverse steps are missing"};
-    }
   });
 }
 
