@@ -338,6 +338,9 @@ lbmx_status lbmx_stream_copy_planes(int planes, size_t nodes, int iters, double*
 lbmx_status lbmx_stream_copy_planes16(int planes, size_t nodes, int iters, double* gbs);
 /* Number of visible HIP devices (0 when the runtime finds none); no handle needed. */
 lbmx_status lbmx_device_count(int* count);
+/* Forward and reverse steps (either may be NULL) that one launch of a forward run or gradient
+   covers; 1: every sweep is a launch of its own. */
+lbmx_status lbmx_steps_per_launch(lbmx_solver* s, int* forward, int* reverse);
 /* Bytes of device memory held by the handle (state, adjoint, checkpoints). */
 lbmx_status lbmx_device_bytes(lbmx_solver* s, size_t* bytes);
 
@@ -370,22 +373,29 @@ lbmx_status lbmx_batch_checkpoint_config(lbmx_batch* b, int nslots);
 /* placement of the shared schedule's checkpoints (lbmx_checkpoint_mode) */
 lbmx_status lbmx_batch_checkpoint_mode(lbmx_batch* b, int mode);
 /* rows of the 64-wide workgroup tile of the batched sweeps: 1, 2 or 4 (default 4), with the
-   forward of 2 and 4 rows taking two nodes per thread */
+   forward of 2 and 4 rows taking two nodes per thread. Once a tile is set, every sweep of a
+   gradient is a launch of its own with that tile; without, 2D batches take several steps per
+   launch where that is faster (lbmx_batch_steps_per_launch). */
 lbmx_status lbmx_batch_set_tile_rows(lbmx_batch* b, int rows);
 /* the same with the forward's pairing chosen: paired != 0 takes rows y and y + rows/2 in one
    thread (2 and 4 rows), paired = 0 one node per thread. Results do not depend on the shape. */
 lbmx_status lbmx_batch_set_tile(lbmx_batch* b, int rows, int paired);
-/* the tile shape in use (set, or chosen by lbmx_batch_autotune); *paired = 0 for 1 row */
+/* the tile shape of the sweeps that are a launch of their own (set, or chosen by
+   lbmx_batch_autotune); *paired = 0 for 1 row */
 lbmx_status lbmx_batch_get_tile(lbmx_batch* b, int* rows, int* paired);
+/* forward and reverse steps (either may be NULL) that one launch of the next gradient covers;
+   1: every sweep is a launch of its own, with the tile of lbmx_batch_get_tile */
+lbmx_status lbmx_batch_steps_per_launch(lbmx_batch* b, int* forward, int* reverse);
 /* enable != 0: the first lbmx_batch_gradient captures its whole launch sequence into a HIP
    graph and later calls with the same steps, slots, tile height and buffers replay it (designs
    may change in between; they are read from the same device arrays). Forward/reverse phase
    times are then not separated in the stats. */
 lbmx_status lbmx_batch_set_graph(lbmx_batch* b, int enable);
 /* Autotuner: times nsweeps batched forward + adjoint sweeps for each tile shape (height 1, 2 or
-   4; the forward of 2 and 4 rows paired or not), keeps the fastest; *rows = chosen height
+   4; the forward of 2 and 4 rows paired or not) and as launches of several steps, keeps the
+   fastest (lbmx_batch_steps_per_launch gives the kind); *rows = chosen height
    (lbmx_batch_get_tile gives the pairing), ms[3] (may be NULL) = ms per forward+adjoint sweep
-   pair for heights 1, 2, 4, each with its better pairing. The members' current states, adjoints and dJ/dgamma arrays are discarded:
+   pair, one step per launch, for heights 1, 2, 4, each with its better pairing. The members' current states, adjoints and dJ/dgamma arrays are discarded:
    until their next gradient, lbmx_get_sensitivity and the other sensitivity reads on a member
    return LBMX_ERR_STATE. */
 lbmx_status lbmx_batch_autotune(lbmx_batch* b, int nsweeps, int* rows, double* ms);

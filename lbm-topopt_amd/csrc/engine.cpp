@@ -1073,6 +1073,7 @@ struct Batch {
   hipStream_t stream = nullptr;
   int ty = kTileY;         // rows of the workgroup tile
   bool pair = true;        // forward of a 2- or 4-row tile: two nodes per thread
+  bool tile_set = false;   // that tile for every sweep: one step per launch
   int nslots = 64;
   int ckpt_mode = LBMX_CHECKPOINT_DYNAMIC;
   int nblocks = 0;
@@ -1164,6 +1165,22 @@ struct Batch {
     return g;
   }
 
+  // steps per launch and tile rows of a gradient pass (dir: 0 forward, 1 reverse)
+  StepsShape shape_of(int dir) const {
+    if (tile_set || !m[0]->steps_possible()) return {1, 1};
+    long long nodes = 0;
+    size_t pieces = 0;
+    for (const Engine* e : m) {
+      nodes += e->N;
+      pieces = std::max(pieces, e->bcs.size());
+    }
+    return lbmx::steps_shape(m[0]->d, dir, (int)pieces, nodes, [&](int H) {
+      long long n = 0;
+      for (const Engine* e : m) n += (long long)((e->d.nx + kTileX - 1) / kTileX) * ((e->d.ny + H - 1) / H);
+      return n;
+    });
+  }
+
   // instance table, workgroup map and member device arrays for the current tile height
   void build() {
     inst.clear();
@@ -1171,18 +1188,9 @@ struct Batch {
     nblocks = 0;
     tf_stride = 1;
     size_t st = 0, lt = 0;
-    long long nodes = 0;
-    for (Engine* e : m) nodes += e->N;
     std::vector<int> steps_map[2];
-    size_t pieces = 0;
-    for (Engine* e : m) pieces = std::max(pieces, e->bcs.size());
-    auto tiles = [&](int H) {
-      long long n = 0;
-      for (Engine* e : m) n += (long long)((e->d.nx + kTileX - 1) / kTileX) * ((e->d.ny + H - 1) / H);
-      return n;
-    };
     for (int dir = 0; dir < 2; ++dir) {
-      steps[dir] = m[0]->steps_possible() ? lbmx::steps_shape(m[0]->d, dir, (int)pieces, nodes, tiles) : StepsShape{1, 1};
+      steps[dir] = shape_of(dir);
       steps_blocks[dir] = 0;
     }
     for (size_t i = 0; i < m.size(); ++i) {
@@ -1436,19 +1444,26 @@ struct Batch {
   }
 
   // Times nsweeps batched forward and adjoint sweeps for each tile shape (height 1, 2 or 4;
-  // the forward of 2 and 4 rows paired or not) and keeps the fastest. ms_out[h] (heights 1, 2,
-  // 4) receives the better pairing of each height.
+  // the forward of 2 and 4 rows paired or not) and, where the batch can take several steps per
+  // launch, those launches; keeps the fastest. ms_out[h] (heights 1, 2, 4) receives the better
+  // pairing of each height, one step per launch.
   int autotune(int nsweeps, double* ms_out) {
     if (nsweeps < 1) throw Error{LBMX_ERR_ARG, "nsweeps must be >= 1"};
     const int cand_ty[5] = {1, 2, 4, 2, 4};
     const bool cand_pair[5] = {true, true, true, false, false};
-    double best = 1e300;
-    int best_ty = ty;
-    bool best_pair = pair;
-    if (ms_out)
-      for (int h = 0; h < 3; ++h) ms_out[h] = 1e300;
+    double one[5][2], several[2] = {0, 0};  // ms of a step, by direction
+    tile_set = false;
     EventPair ev;
-    hipEvent_t e0 = ev.e0, e1 = ev.e1;
+    auto timed = [&](int launches, auto&& f) {
+      f();  // warm-up
+      HIP_OK(hipEventRecord(ev.e0, stream));
+      for (int k = 0; k < launches; ++k) f();
+      HIP_OK(hipEventRecord(ev.e1, stream));
+      HIP_OK(hipEventSynchronize(ev.e1));
+      float ms = 0;
+      HIP_OK(hipEventElapsedTime(&ms, ev.e0, ev.e1));
+      return double(ms) / launches;
+    };
     for (int c = 0; c < 5; ++c) {
       ty = cand_ty[c];
       pair = cand_pair[c];
@@ -1456,7 +1471,7 @@ struct Batch {
       ensure_pool(2);
       lam_a.ensure(lam_total);
       lam_b.ensure(lam_total);
-      upload_tfac(1);
+      upload_tfac(kMaxSteps);
       const double u0[3] = {0, 0, 0};
       init_all(pool[0]->p, 1.0, u0, 0.0);
       zero_async(lam_a.p, lam_total, stream);
@@ -1464,32 +1479,51 @@ struct Batch {
       for (auto& I : inst) zero_async(I.sens, (size_t)I.g.N * 8, stream);
       void* a = pool[0]->p;
       void* b = pool[1]->p;
-      HIP_OK(launch(0, a, b, nullptr, nullptr, 1, false));  // warm-up
-      HIP_OK(hipEventRecord(e0, stream));
-      for (int k = 0; k < nsweeps; ++k) {
+      one[c][0] = timed(nsweeps, [&] {
         HIP_OK(launch(0, a, b, nullptr, nullptr, 1, false));
         std::swap(a, b);
-      }
+      });
       void* li = lam_a.p;
       void* lo = lam_b.p;
-      for (int k = 0; k < nsweeps; ++k) {
+      one[c][1] = timed(nsweeps, [&] {
         HIP_OK(launch(1, a, nullptr, li, lo, 1, true));
         std::swap(li, lo);
-      }
-      HIP_OK(hipEventRecord(e1, stream));
-      HIP_OK(hipEventSynchronize(e1));
-      float ms = 0;
-      HIP_OK(hipEventElapsedTime(&ms, e0, e1));
-      const int h = ty == 1 ? 0 : ty == 2 ? 1 : 2;
-      if (ms_out) ms_out[h] = std::min(ms_out[h], double(ms) / nsweeps);
-      if (ms < best) {
-        best = ms;
-        best_ty = ty;
-        best_pair = pair;
+      });
+      for (int dir = 0; c == 0 && dir < 2; ++dir) {
+        const int K = steps[dir].K;
+        if (K == 1) continue;
+        several[dir] = timed((nsweeps + K - 1) / K, [&] {
+                         void* bufs[kMaxSteps] = {};
+                         if (dir) std::fill(bufs, bufs + K, a);
+                         else bufs[K - 1] = b;
+                         HIP_OK(launch_steps(dir, a, bufs, li, lo, dir ? K : 1, K, dir != 0));
+                         if (dir) std::swap(li, lo);
+                         else std::swap(a, b);
+                       }) / K;
       }
     }
-    ty = best_ty;
-    pair = best_pair;
+    int best_one = 0, best_several = 0;
+    double t_one = 1e300, t_several = 1e300;
+    for (int c = 0; c < 5; ++c) {
+      const double o = one[c][0] + one[c][1];
+      const double v = (steps[0].K > 1 ? several[0] : one[c][0]) + (steps[1].K > 1 ? several[1] : one[c][1]);
+      if (o < t_one) {
+        t_one = o;
+        best_one = c;
+      }
+      if (v < t_several) {
+        t_several = v;
+        best_several = c;
+      }
+    }
+    if (ms_out) {
+      ms_out[0] = one[0][0] + one[0][1];
+      for (int h = 1; h < 3; ++h) ms_out[h] = std::min(one[h][0] + one[h][1], one[h + 2][0] + one[h + 2][1]);
+    }
+    tile_set = t_one < t_several;
+    const int best = tile_set || (steps[0].K > 1 && steps[1].K > 1) ? best_one : best_several;
+    ty = cand_ty[best];
+    pair = cand_pair[best];
     // the timed sweeps overwrote every member's state and accumulated into its dJ/dgamma array
     for (Engine* e : m) {
       e->state_kind = -1;
@@ -1500,7 +1534,8 @@ struct Batch {
   }
 
   size_t device_bytes() const {
-    size_t b = inst_dev.bytes + blk_dev.bytes + tfac_dev.bytes + lam_a.bytes + lam_b.bytes;
+    size_t b = inst_dev.bytes + blk_dev.bytes + steps_blk_dev[0].bytes + steps_blk_dev[1].bytes + tfac_dev.bytes +
+               lam_a.bytes + lam_b.bytes;
     for (auto& p : pool) b += p->bytes;
     return b;
   }
@@ -1877,6 +1912,7 @@ lbmx_status lbmx_batch_set_tile_rows(lbmx_batch* b, int rows) {
   }
   b->b->ty = rows;
   b->b->pair = true;
+  b->b->tile_set = true;
   return LBMX_OK;
 }
 
@@ -1888,6 +1924,7 @@ lbmx_status lbmx_batch_set_tile(lbmx_batch* b, int rows, int paired) {
   }
   b->b->ty = rows;
   b->b->pair = paired != 0;
+  b->b->tile_set = true;
   return LBMX_OK;
 }
 
@@ -1895,6 +1932,13 @@ lbmx_status lbmx_batch_get_tile(lbmx_batch* b, int* rows, int* paired) {
   CHECK_BATCH(b);
   if (rows) *rows = b->b->ty;
   if (paired) *paired = (b->b->ty > 1 && b->b->pair) ? 1 : 0;
+  return LBMX_OK;
+}
+
+lbmx_status lbmx_batch_steps_per_launch(lbmx_batch* b, int* forward, int* reverse) {
+  CHECK_BATCH(b);
+  if (forward) *forward = b->b->shape_of(0).K;
+  if (reverse) *reverse = b->b->shape_of(1).K;
   return LBMX_OK;
 }
 
@@ -1944,6 +1988,13 @@ lbmx_status lbmx_time_sweeps(lbmx_solver* s, int kind, int nsweeps, double* ms) 
   CHECK_HANDLE(s);
   if (!ms) { lbmx::g_last_error = "null argument"; return LBMX_ERR_ARG; }
   return guarded([&] { *ms = s->e->time_sweeps(kind, nsweeps); });
+}
+
+lbmx_status lbmx_steps_per_launch(lbmx_solver* s, int* forward, int* reverse) {
+  CHECK_HANDLE(s);
+  if (forward) *forward = s->e->steps_shape(0).K;
+  if (reverse) *reverse = s->e->steps_shape(1).K;
+  return LBMX_OK;
 }
 
 lbmx_status lbmx_device_bytes(lbmx_solver* s, size_t* bytes) {

@@ -188,6 +188,8 @@ def library():
         "lbmx_batch_set_tile": [C.c_void_p, C.c_int, C.c_int],
         "lbmx_design_change_noalloc": [dp, dp, C.c_longlong, dp, C.c_void_p],
         "lbmx_batch_get_tile": [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int)],
+        "lbmx_batch_steps_per_launch": [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int)],
+        "lbmx_steps_per_launch": [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int)],
         "lbmx_batch_set_graph": [C.c_void_p, C.c_int],
         "lbmx_batch_autotune": [C.c_void_p, C.c_int, P(C.c_int), dp],
         "lbmx_batch_gradient": [C.c_void_p, C.c_int, C.c_double, dp, C.c_double, dp, P(dp)],
@@ -262,7 +264,7 @@ EXPORTED = ["lbmx_create", "lbmx_destroy", "lbmx_set_stream", "lbmx_last_error",
             "lbmx_dmda_global_to_natural", "lbmx_dmda_natural_to_global", "lbmx_checkpoint_mode",
             "lbmx_checkpoint_simulate_mode", "lbmx_batch_checkpoint_mode",
             "lbmx_batch_set_tile", "lbmx_batch_get_tile", "lbmx_add_boundary_table",
-            "lbmx_design_change_noalloc"]
+            "lbmx_design_change_noalloc", "lbmx_steps_per_launch", "lbmx_batch_steps_per_launch"]
 
 
 def checkpoint_simulate(nslots, nsteps, mode=CHECKPOINT_DYNAMIC):
@@ -537,6 +539,12 @@ class Solver:
             out.append((v[0], tuple(v[1:4]), tuple(v[4:10])))
         return out
 
+    def steps_per_launch(self):
+        """(forward, reverse) steps that one launch of a forward run or gradient covers."""
+        f, r = C.c_int(0), C.c_int(0)
+        _check(self.lib.lbmx_steps_per_launch(self.h, C.byref(f), C.byref(r)))
+        return f.value, r.value
+
     def device_bytes(self):
         b = C.c_size_t(0)
         _check(self.lib.lbmx_device_bytes(self.h, C.byref(b)))
@@ -577,16 +585,23 @@ class Batch:
         _check(self.lib.lbmx_batch_set_tile(self.h, rows, 1 if paired else 0))
 
     def tile(self):
-        """(rows, paired) of the tile shape in use."""
+        """(rows, paired) of the tile shape of the sweeps that are a launch of their own."""
         r, p = C.c_int(0), C.c_int(0)
         _check(self.lib.lbmx_batch_get_tile(self.h, C.byref(r), C.byref(p)))
         return r.value, bool(p.value)
+
+    def steps_per_launch(self):
+        """(forward, reverse) steps that one launch of the next gradient covers."""
+        f, r = C.c_int(0), C.c_int(0)
+        _check(self.lib.lbmx_batch_steps_per_launch(self.h, C.byref(f), C.byref(r)))
+        return f.value, r.value
 
     def set_graph(self, enable=True):
         _check(self.lib.lbmx_batch_set_graph(self.h, 1 if enable else 0))
 
     def autotune(self, nsweeps=10):
-        """Returns (chosen tile rows, ms per forward+adjoint sweep pair for rows 1, 2, 4)."""
+        """Returns (chosen tile rows, ms per forward+adjoint sweep pair for rows 1, 2, 4, one step per
+        launch); steps_per_launch() says whether launches of several steps were faster."""
         r = C.c_int(0)
         ms = (C.c_double * 3)()
         _check(self.lib.lbmx_batch_autotune(self.h, nsweeps, C.byref(r), ms))
