@@ -321,7 +321,8 @@ typedef struct {
   long long recompute_sweeps; /* forward sweeps re-run in reverse phases                 */
 } lbmx_stats;
 lbmx_status lbmx_get_stats(lbmx_solver* s, lbmx_stats* st);
-/* Times nsweeps back-to-back sweeps with HIP events on the handle's stream. kind 0: forward
+/* Times nsweeps back-to-back sweeps with HIP events on the handle's stream, in the launches that a
+   forward run or a gradient makes of them (lbmx_steps_per_launch). kind 0: forward
    sweeps from the current state (the state advances, objective accumulation on); kind 1:
    adjoint sweeps reading the current state as p_{t-1} with ping-ponged adjoint buffers.
    *ms = total device time of the sweeps. */

@@ -740,15 +740,9 @@ struct Engine {
     return s;
   }
 
-  void forward(int nsteps, double* J) {
-    require_state();
-    if (nsteps < 0) throw Error{LBMX_ERR_ARG, "nsteps must be >= 0"};
-    check_time_tables((long long)t + nsteps);
-    prepare();
-    bool with_obj = J && obj_set && obj.nterm > 0;
-    if (with_obj) zero_acc();
-    auto t0 = std::chrono::steady_clock::now();
-    // (the last step by itself: its input p_{t-1} stays available)
+  // the launches of nsteps forward steps from the current state; the last step by itself: its
+  // input p_{t-1} stays available
+  void advance(int nsteps, bool with_obj) {
     const int most = steps_shape(0).K;
     for (int left = nsteps; left > 0;) {
       const int k = left == 1 ? 1 : std::min(left - 1, most);
@@ -761,6 +755,17 @@ struct Engine {
       state_kind = 0;
     }
     stats.fwd_sweeps += nsteps;
+  }
+
+  void forward(int nsteps, double* J) {
+    require_state();
+    if (nsteps < 0) throw Error{LBMX_ERR_ARG, "nsteps must be >= 0"};
+    check_time_tables((long long)t + nsteps);
+    prepare();
+    bool with_obj = J && obj_set && obj.nterm > 0;
+    if (with_obj) zero_acc();
+    auto t0 = std::chrono::steady_clock::now();
+    advance(nsteps, with_obj);
     double Jv = with_obj ? reduce_acc() : 0.0;
     HIP_OK(hipStreamSynchronize(stream));
     stats.forward_phase_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1009,15 +1014,8 @@ struct Engine {
       const bool with_obj = obj_set && obj.nterm > 0;
       if (with_obj) zero_acc();
       HIP_OK(hipEventRecord(e0, stream));
-      for (int k = 0; k < nsweeps; ++k) {
-        FwdArgs a = fwd_args(cur, prev, t + 1, with_obj);
-        HIP_OK(run_fwd(a));
-        std::swap(cur, prev);
-        ++t;
-      }
+      advance(nsweeps, with_obj);
       HIP_OK(hipEventRecord(e1, stream));
-      state_kind = 0;
-      stats.fwd_sweeps += nsweeps;
     } else {
       lam_a.ensure(lam_bytes());
       lam_b.ensure(lam_bytes());
@@ -1031,10 +1029,14 @@ struct Engine {
       void* lin = lam_a.p;
       void* lout = lam_b.p;
       HIP_OK(hipEventRecord(e0, stream));
-      for (int k = 0; k < nsweeps; ++k) {
-        AdjArgs a = adj_args(cur, lin, lout, std::max(1, t), oa);
-        HIP_OK(run_adj(a));
+      const int most = steps_shape(1).K;
+      for (int left = nsweeps; left > 0;) {
+        const int k = std::min(left, most);
+        void* state[kMaxSteps];
+        std::fill(state, state + k, cur);
+        HIP_OK(run_adj_steps(state, lin, lout, std::max(1, t), k, oa));
         std::swap(lin, lout);
+        left -= k;
       }
       HIP_OK(hipEventRecord(e1, stream));
       stats.adj_sweeps += nsweeps;

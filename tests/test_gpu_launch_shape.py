@@ -58,3 +58,38 @@ def test_autotune_weighs_launches_of_several_steps(lbmx_mod):
     J1, g1 = run(b)
     assert list(J1) == list(J) and all(np.array_equal(x, y) for x, y in zip(g, g1))
     b.close()
+
+
+def test_time_sweeps_times_the_launches_of_a_pass(lbmx_mod):
+    """time_sweeps makes the launches that forward and gradient make: the device time of n sweeps
+    is within a quarter of the pass's wall time (a launch per step takes 1.6 times it here), and
+    the state it leaves is that of forward."""
+    n, nx, ny = 600, 256, 128
+    s = lbmx.Solver(lbmx.make_desc(nx, ny, lattice=lbmx.D2Q9, collision=lbmx.MRT, design=lbmx.DESIGN_BRINKMAN,
+                                   precision=lbmx.FP64, omega=1.3, interp_q=0.1, alpha_max=0.1))
+    workloads.channel2d(s, nx, ny, time_const=1.0 / n)
+    s.set_design(workloads.design_field(nx, ny, 1, seed=3))
+    assert min(s.steps_per_launch()) > 1
+    s.init_equilibrium(u0=(0.02, 0.0, 0.0))
+    s.forward(n)
+    after = s.get_state()
+    s.init_equilibrium(u0=(0.02, 0.0, 0.0))
+    s.time_sweeps(0, n)
+    assert s.timestep() == n and np.array_equal(s.get_state(), after)
+    wall, timed = [], []
+    for _ in range(3):
+        s.init_equilibrium(u0=(0.02, 0.0, 0.0))
+        s.forward(n)
+        wall.append(s.stats()["forward_phase_ms"])
+        timed.append(s.time_sweeps(0, n))
+    assert min(timed) < 1.25 * min(wall)
+    s.checkpoint_config(0)
+    wall, timed = [], []
+    for _ in range(3):
+        s.gradient(n, u0=(0.02, 0.0, 0.0))
+        wall.append(s.stats()["reverse_phase_ms"])
+        s.init_equilibrium(u0=(0.02, 0.0, 0.0))
+        s.forward(8)
+        timed.append(s.time_sweeps(1, n))
+    assert min(timed) < 1.25 * min(wall)
+    s.close()
