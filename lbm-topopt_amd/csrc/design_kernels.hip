@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "design_cone.hpp"
+#include "design_cone_shape.hpp"
 #include "lbmx_launch.h"
 
 namespace lbmx {
@@ -11,12 +12,6 @@ namespace lbmx {
 namespace {
 
 constexpr int kMaxR = 16;
-
-// ---- cone of any radius ----
-constexpr int kConeTX = 64;   // outputs along x per workgroup (one wave wide)
-constexpr int kConeWY = 4;    // waves per workgroup, stacked along y
-constexpr int kConeKY = 4;    // outputs per thread along y (four named sums in k_cone)
-constexpr int kConeTY = kConeWY * kConeKY;  // outputs along y per workgroup
 
 // LDS bytes of one workgroup: the input region of one plane and that plane's cone weights
 inline size_t cone_lds_bytes(int R) {
@@ -179,16 +174,12 @@ inline Box6 box6(const int b[6]) {
 
 }  // namespace
 
-// Radii up to these have a kernel of their own (2D: 2 x 2 outputs per lane, 3D: 2 x 4 x 4).
-// The unrolled taps fill about 30 KB of the 64 KB instruction cache at radius 12 in 2D and all
-// of it at radius 3 in 3D (32 x 123 taps per lane); larger radii take the kernel of any radius.
-constexpr int kConeFixed2D = 12;
-constexpr int kConeFixed3D = 3;
-
 hipError_t launch_cone(const ConeArgs& a, hipStream_t s) {
   if (a.R < 1 || a.R > kMaxR || a.nx < 1 || a.ny < 1 || a.nz < 1) return hipErrorInvalidValue;
-  if (a.nz == 1 && a.R <= kConeFixed2D) return a.R <= 8 ? launch_cone_2d_small(a, s) : launch_cone_2d_large(a, s);
-  if (a.nz > 1 && a.R <= kConeFixed3D) return launch_cone_3d_small(a, s);
+  if (cone_fixed_radius(a.nx, a.ny, a.nz, a.R, a.transposed != 0)) {
+    if (a.nz > 1) return launch_cone_3d_small(a, s);
+    return a.R <= 8 ? launch_cone_2d_small(a, s) : launch_cone_2d_large(a, s);
+  }
   dim3 grid((a.nx + kConeTX - 1) / kConeTX, (a.ny + kConeTY - 1) / kConeTY, a.nz);
   hipLaunchKernelGGL(k_cone, grid, dim3(kConeTX * kConeWY), cone_lds_bytes(a.R), s, a);
   return hipGetLastError();

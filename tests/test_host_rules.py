@@ -32,3 +32,7 @@ def test_checkpoint_count_streams():
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120, env=env)
     assert r.returncode == 0, r.stderr[-2000:]
     assert int(r.stdout.split()[-1]) < 8 * 1024  # KiB; 300000 steps in lists take tens of MiB
+
+
+def test_cone_kernel_choice(tmp_path):
+    run_program(tmp_path, "cone_shape_check")
