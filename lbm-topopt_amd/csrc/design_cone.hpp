@@ -35,11 +35,12 @@ __device__ __forceinline__ double cone_input(const ConeArgs& a, int x, int y, in
 }
 
 // the input as the cone reads it: 0 outside the grid and, transposed, outside the box (only
-// rows inside the box carry cone weights)
+// rows inside the box carry cone weights); MAPPED: the input is the mapped design
+template <bool MAPPED, bool TR>
 __device__ __forceinline__ double cone_tile_value(const ConeArgs& a, int x, int y, int z) {
   if (x < 0 || x >= a.nx || y < 0 || y >= a.ny) return 0.0;
-  if (a.transposed && !in_box(x, y, z, a.box)) return 0.0;
-  return cone_input(a, x, y, z);
+  if (TR && !in_box(x, y, z, a.box)) return 0.0;
+  return MAPPED ? cone_input(a, x, y, z) : a.in[node(a, x, y, z)];
 }
 
 // tanh(x) = E / (E + 2) with E = exp(2|x|) - 1: 2|x| = n ln 2 + r in two parts, E on r from

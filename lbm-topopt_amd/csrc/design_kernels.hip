@@ -22,7 +22,10 @@ inline size_t cone_lds_bytes(int R) {
 // One workgroup: a 64 x 16 tile of outputs in one z plane. For each in-grid plane z + dz the
 // (64 + 2R) x (16 + 2R) input region and the plane's (2R + 1)^2 weights are staged in LDS;
 // then for each tap row (dy) and tap (dx) one weight is read and applied to the thread's four
-// outputs (four independent sums, each in ascending (dz, dy, dx) order).
+// outputs (four independent sums, each in ascending (dz, dy, dx) order). MAPPED: the input is the
+// mapped design (a.design); a test of that per staged value costs 2 to 4% of a call (101x47x53,
+// radius 4, transposed: 87 us with it, 82 us without).
+template <bool MAPPED, bool TR>
 __global__ __launch_bounds__(256) void k_cone(ConeArgs a) {
 #pragma clang fp contract(off)
   extern __shared__ double lds[];
@@ -48,7 +51,7 @@ __global__ __launch_bounds__(256) void k_cone(ConeArgs a) {
     acc[k] = 0.0;
     const bool valid = x < a.nx && y < a.ny;
     mine[k] = valid && in_box(x, y, z, a.box);
-    own[k] = valid && a.transposed ? cone_input(a, x, y, z) : 0.0;
+    own[k] = TR && valid ? a.in[node(a, x, y, z)] : 0.0;
   }
 
   for (int dz = -R; dz <= R; ++dz) {
@@ -56,7 +59,7 @@ __global__ __launch_bounds__(256) void k_cone(ConeArgs a) {
     if (zz < 0 || zz >= a.nz) continue;  // uniform over the workgroup
     __syncthreads();
     for (int idx = threadIdx.x; idx < W * H; idx += blockDim.x)
-      tile[idx] = cone_tile_value(a, x0 - R + idx % W, y0 - R + idx / W, zz);
+      tile[idx] = cone_tile_value<MAPPED, TR>(a, x0 - R + idx % W, y0 - R + idx / W, zz);
     const double* wz = a.wt + (size_t)(dz + R) * S * S;
     for (int idx = threadIdx.x; idx < S * S; idx += blockDim.x) wl[idx] = wz[idx];
     __syncthreads();
@@ -102,7 +105,7 @@ __global__ __launch_bounds__(256) void k_cone(ConeArgs a) {
         taps(-r, 0);
         // the diagonal entry: cone weight for a row in the box, 1 for an identity row
         const double wv = w[0];
-        if (a.transposed) {
+        if constexpr (TR) {
           s0 = s0 + (mine[0] ? wv : 1.0) * own[0];
           s1 = s1 + (mine[1] ? wv : 1.0) * own[1];
           s2 = s2 + (mine[2] ? wv : 1.0) * own[2];
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(256) void k_cone(ConeArgs a) {
     const int y = y0 + ty + kConeWY * k;
     if (x < a.nx && y < a.ny) {
       double v = 0.0, p = 0.0;
-      cone_finish(a, x, y, z, acc[0], a.transposed ? 1.0 : cone_second(a, x, y, z), v, p);
+      cone_finish(a, x, y, z, acc[0], TR ? 1.0 : cone_second(a, x, y, z), v, p);
       cone_store(a, x, y, z, v, p);
     }
     for (int i = 1; i < kConeKY; ++i) acc[i - 1] = acc[i];
@@ -181,7 +184,10 @@ hipError_t launch_cone(const ConeArgs& a, hipStream_t s) {
     return a.R <= 8 ? launch_cone_2d_small(a, s) : launch_cone_2d_large(a, s);
   }
   dim3 grid((a.nx + kConeTX - 1) / kConeTX, (a.ny + kConeTY - 1) / kConeTY, a.nz);
-  hipLaunchKernelGGL(k_cone, grid, dim3(kConeTX * kConeWY), cone_lds_bytes(a.R), s, a);
+  const dim3 block(kConeTX * kConeWY);
+  if (a.transposed) hipLaunchKernelGGL((k_cone<false, true>), grid, block, cone_lds_bytes(a.R), s, a);
+  else if (a.design) hipLaunchKernelGGL((k_cone<true, false>), grid, block, cone_lds_bytes(a.R), s, a);
+  else hipLaunchKernelGGL((k_cone<false, false>), grid, block, cone_lds_bytes(a.R), s, a);
   return hipGetLastError();
 }
 
