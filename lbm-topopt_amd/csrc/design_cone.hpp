@@ -8,6 +8,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "design_cone_shape.hpp"
 #include "lbmx_device.hpp"
 #include "lbmx_launch.h"
 
@@ -400,6 +401,7 @@ hipError_t cone_fixed(const ConeArgs& a, hipStream_t s) {
 // the 2D kernel of radius a.R, searched from R0 to R1
 template <int R0, int R1>
 hipError_t cone_2d(const ConeArgs& a, hipStream_t s) {
+  static_assert(ConeTile<R0, 2, 1>::TY == kConeFixedTY2D, "cone_fixed_radius counts workgroups of this height");
   if constexpr (R0 <= R1) {
     if (a.R == R0) return cone_fixed<R0, 2, 1, false>(a, s);
     return cone_2d<R0 + 1, R1>(a, s);

@@ -15,6 +15,8 @@ constexpr int kConeTY = kConeWY * kConeKY;  // outputs along y per workgroup
 // instruction cache (32 x 123 taps per lane).
 constexpr int kConeFixed2D = 12;
 constexpr int kConeFixed3D = 3;
+constexpr int kConeFixedTY2D = 8;  // outputs along y per workgroup of the 2D kernel
+constexpr int kMaxGridY = 65535;   // most workgroups along y of a launch
 
 // Whether the kernel of the radius runs. In 2D it does on every grid (0.74 to 0.97 of the other's
 // time from 48x24 to 2049x1025, also on grids 30 and 70 wide). A 3D lane sums 32 outputs one plane
@@ -24,7 +26,8 @@ constexpr int kConeFixed3D = 3;
 // (plain and projecting) near 3500, 1500 and 1100 for radii 1, 2 and 3, transposed near 1600, 900
 // and 700.
 constexpr bool cone_fixed_radius(int nx, int ny, int nz, int R, bool transposed) {
-  if (nz == 1) return R <= kConeFixed2D;
+  // (a 2D grid of more than 524280 rows has too many workgroups along y for the low tile)
+  if (nz == 1) return R <= kConeFixed2D && (ny + kConeFixedTY2D - 1) / kConeFixedTY2D <= kMaxGridY;
   if (R > kConeFixed3D) return false;
   constexpr long long least[2][kConeFixed3D] = {{3500, 1500, 1100}, {1600, 900, 700}};
   const long long blocks = (long long)((nx + kConeTX - 1) / kConeTX) * ((ny + kConeTY - 1) / kConeTY) * nz;

@@ -26,6 +26,10 @@ int main() {
       for (int r = R; r <= 12; r += 3) expect(true, 48, 24, 1, r, tr);
     }
   expect(false, 48, 24, 1, 13, false);
+  // a launch has at most 65535 workgroups along y
+  expect(true, 3, 524280, 1, 2, false);
+  expect(false, 3, 524281, 1, 2, false);
+  expect(false, 3, 1048560, 1, 12, true);
   if (!fails) std::printf("RESULT OK\n");
   return fails != 0;
 }

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 CASES = [((129, 17, nz), (1, 127, 2, 15, 1, nz - 2), R)
          for R, sizes in ((1, (266, 267, 583, 587)), (2, (149, 151, 247, 251)), (3, (115, 117, 183, 185))) for nz in sizes]
 CASES += [((37, 5, 2), (30, 36, 0, 4, 0, 1), 3), ((16, 16, 16), (0, 15, 0, 15, 0, 15), 2)]
+CASES += [((3, ny, 1), (0, 2, 1, ny - 2, 0, 0), 2) for ny in (524280, 524281, 700001)]  # tall 2D grids
 
 
 @pytest.mark.parametrize("dims,fbox,R", CASES)
