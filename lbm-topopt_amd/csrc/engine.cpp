@@ -39,6 +39,7 @@ static void zero_async(void* p, size_t bytes, hipStream_t s) { HIP_OK(fill_zero(
 
 struct Engine {
   lbmx_desc d{};
+  mutable int num_cus = 0;          // CUs of the device (0: not asked yet)
   int Q = 0, D = 0;
   long long N = 0;
   bool inc = true;
@@ -554,9 +555,18 @@ struct Engine {
   // Several steps per launch: 2D lattices without Neumann pieces, whose transfers between nodes
   // run between the sweeps. dir: 0 forward, 1 reverse.
   bool steps_possible() const { return D == 2 && nside_count == 0; }
+  int cus() const {
+    if (num_cus == 0) {
+      int dev = 0;
+      if (hipGetDevice(&dev) != hipSuccess ||
+          hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || num_cus < 1)
+        num_cus = 256;
+    }
+    return num_cus;
+  }
   StepsShape steps_shape(int dir) const {
     if (!steps_possible()) return {1, 1};
-    return lbmx::steps_shape(d, dir, (int)bcs.size(), N, [&](int H) {
+    return lbmx::steps_shape(d, dir, (int)bcs.size(), N, cus(), [&](int H) {
       return (long long)((d.nx + kTileX - 1) / kTileX) * ((d.ny + H - 1) / H);
     });
   }
@@ -1176,7 +1186,7 @@ struct Batch {
       nodes += e->N;
       pieces = std::max(pieces, e->bcs.size());
     }
-    return lbmx::steps_shape(m[0]->d, dir, (int)pieces, nodes, [&](int H) {
+    return lbmx::steps_shape(m[0]->d, dir, (int)pieces, nodes, m[0]->cus(), [&](int H) {
       long long n = 0;
       for (const Engine* e : m) n += (long long)((e->d.nx + kTileX - 1) / kTileX) * ((e->d.ny + H - 1) / H);
       return n;

@@ -1,20 +1,22 @@
 // Shape of a launch that takes tiles of a 2D field through several steps (lbmx_steps.hpp): the
-// steps K and the tile's rows H, by what such a workgroup takes and by how many there are.
+// steps K and the tile's rows H, by what such a workgroup takes and by how many there are. No
+// device code: the functions are constant expressions, which the kernels use too.
 #pragma once
-#include "lbmx_device.hpp"
+#include "lbmx.h"
+#include "lbmx_common.h"
 
 namespace lbmx {
 
 // dynamic LDS of a launch: boundary pieces, their K time factors, then the field(s)
-__host__ __device__ constexpr size_t steps_pieces_bytes(int nbc, int K) {
+constexpr size_t steps_pieces_bytes(int nbc, int K) {
   return ((size_t)nbc * (sizeof(DevBC) + (size_t)K * sizeof(double)) + 15) & ~(size_t)15;
 }
-__host__ __device__ constexpr int steps_cells(int K, int H) { return (kTileX + 2 * (K - 1)) * (H + 2 * (K - 1)); }
-__host__ __device__ constexpr size_t steps_field_bytes(int K, int H, int Q, int elem) {
+constexpr int steps_cells(int K, int H) { return (kTileX + 2 * (K - 1)) * (H + 2 * (K - 1)); }
+constexpr size_t steps_field_bytes(int K, int H, int Q, int elem) {
   return (((size_t)steps_cells(K, H) * Q * elem + 15) & ~(size_t)15) * (K > 2 ? 2 : 1);
 }
 // waves of a workgroup: the region's rows, and the columns beside the 64
-__host__ __device__ constexpr int steps_waves(int K, int H) {
+constexpr int steps_waves(int K, int H) {
   const int rows = H + 2 * (K - 1), side = 2 * (K - 1) * rows;
   return rows + (side + kTileX - 1) / kTileX;
 }
@@ -22,13 +24,14 @@ __host__ __device__ constexpr int steps_waves(int K, int H) {
 // workgroup of 16 waves leaves each lane (they spill up to 200 of them, and at 1024 x 512 a
 // reverse step takes 30 us instead of the single-step sweep's 27); with 12 waves they have 168
 // and it takes 21.
-__host__ __device__ constexpr int steps_max_waves(int dir, bool fp64) { return dir == 1 && fp64 ? 12 : 16; }
+constexpr int steps_max_waves(int dir, bool fp64) { return dir == 1 && fp64 ? 12 : 16; }
 
 struct StepsShape {
   int K, H;  // K = 1: the single-step sweeps
 };
 
-// dir: 0 forward, 1 reverse; nodes, blocks(H): of all fields that a launch covers.
+// dir: 0 forward, 1 reverse; nodes, blocks(H): of all fields that a launch covers; cus: CUs of the
+// device (256, or an eighth of them where it is partitioned).
 //
 // A workgroup of this kind fills a CU, so what counts first is whether all of them run at once
 // (at most one per CU). Then a launch's time hardly depends on the tile and more steps per launch
@@ -53,8 +56,7 @@ struct StepsShape {
 // arithmetic of all (FP64 at 1024x512 34.9 and 36.8), and its long polynomials, left to the
 // compiler's fusing, do not come out with the same bits in both kernels.
 template <class Blocks>
-StepsShape steps_shape(const lbmx_desc& d, int dir, int nbc, long long nodes, Blocks&& blocks) {
-  constexpr int kCUs = 256;
+inline StepsShape steps_shape(const lbmx_desc& d, int dir, int nbc, long long nodes, int cus, Blocks&& blocks) {
   constexpr size_t kLds = 160 * 1024;
   const bool fp64 = d.precision == LBMX_FP64, fp32 = d.precision == LBMX_FP32;
   const bool thermal = d.lattice == LBMX_D2Q9_D2Q5, cascaded = d.collision == LBMX_CASCADED;
@@ -66,7 +68,7 @@ StepsShape steps_shape(const lbmx_desc& d, int dir, int nbc, long long nodes, Bl
   };
   for (int K = kMaxSteps; K > 1; --K)
     for (int H = 2; fits(K, H); ++H)
-      if (blocks(H) <= kCUs) return {K, H};
+      if (blocks(H) <= cus) return {K, H};
   if (dir == 0 && !fp64 && !fp32) return {1, 1};
   if (dir == 0 && fp32 && cascaded && nodes > (1ll << 21)) return {1, 1};
   if (dir == 1 && fp64 && thermal && d.design == LBMX_DESIGN_BRINKMAN) return {1, 1};

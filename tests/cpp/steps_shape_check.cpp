@@ -1,0 +1,73 @@
+// Shapes of the launches that take several steps (lbmx_steps_shape.hpp): every one stays within a
+// workgroup's waves and LDS, and the rule. Prints "RESULT OK" at the end.
+#include <cstdio>
+#include <vector>
+
+#include "lbmx_steps_shape.hpp"
+
+using namespace lbmx;
+
+static int fails = 0;
+
+struct Form {
+  int lattice, collision, design, precision;
+};
+
+static StepsShape shape(const Form& f, int dir, int nx, int ny, int nbc = 7, int cus = 256) {
+  lbmx_desc d{};
+  d.lattice = f.lattice;
+  d.collision = f.collision;
+  d.design = f.design;
+  d.precision = f.precision;
+  return steps_shape(d, dir, nbc, (long long)nx * ny, cus, [&](int H) {
+    return (long long)((nx + kTileX - 1) / kTileX) * ((ny + H - 1) / H);
+  });
+}
+
+static void expect(const Form& f, int dir, int nx, int ny, int K, int H, int cus = 256) {
+  const StepsShape s = shape(f, dir, nx, ny, 7, cus);
+  if (s.K == K && (s.H == H || K == 1)) return;
+  std::printf("lattice %d collision %d design %d precision %d dir %d %d x %d on %d CUs: %d steps of %d rows, not %d of %d\n",
+              f.lattice, f.collision, f.design, f.precision, dir, nx, ny, cus, s.K, s.H, K, H);
+  ++fails;
+}
+
+int main() {
+  std::vector<Form> forms;
+  for (int lat : {LBMX_D2Q9, LBMX_D2Q9_D2Q5})
+    for (int coll : {LBMX_BGK, LBMX_MRT, LBMX_CASCADED})
+      for (int des : {LBMX_DESIGN_NONE, LBMX_DESIGN_PBB, LBMX_DESIGN_BRINKMAN})
+        for (int prec : {LBMX_FP64, LBMX_FP32, LBMX_FP16_SHIFTED, LBMX_BF16_SHIFTED})
+          if (lat == LBMX_D2Q9 || coll != LBMX_CASCADED) forms.push_back({lat, coll, des, prec});
+  for (const Form& f : forms)
+    for (int dir : {0, 1})
+      for (int nx : {1, 2, 12, 48, 64, 65, 100, 128, 200, 330, 640, 1024, 2048, 4100})
+        for (int ny : {1, 2, 5, 24, 128, 301, 512, 1024, 4000, 16000})
+          for (int nbc : {0, 1, 4, 7, kMaxBC})
+            for (int cus : {32, 256}) {
+              const StepsShape s = shape(f, dir, nx, ny, nbc, cus);
+              const bool fp64 = f.precision == LBMX_FP64;
+              const int elem = fp64 ? 8 : (f.precision == LBMX_FP32 || dir == 1 ? 4 : 2);
+              const bool ok = s.K == 1 ||
+                              (s.K <= kMaxSteps && s.H >= 2 && steps_waves(s.K, s.H) <= steps_max_waves(dir, fp64) &&
+                               steps_pieces_bytes(nbc, s.K) +
+                                       steps_field_bytes(s.K, s.H, f.lattice == LBMX_D2Q9 ? 9 : 14, elem) <=
+                                   160 * 1024);
+              if (!ok || s.K < 1) {
+                std::printf("%d x %d dir %d, %d pieces: %d steps of %d rows do not fit\n", nx, ny, dir, nbc, s.K, s.H);
+                ++fails;
+              }
+            }
+  const Form mrt64{LBMX_D2Q9, LBMX_MRT, LBMX_DESIGN_BRINKMAN, LBMX_FP64};
+  const Form casc32{LBMX_D2Q9, LBMX_CASCADED, LBMX_DESIGN_PBB, LBMX_FP32};
+  // one round of workgroups: the deepest launch with the fewest rows
+  expect(mrt64, 0, 256, 128, 4, 2);
+  expect(mrt64, 0, 512, 256, 4, 8);
+  expect(mrt64, 1, 512, 256, 2, 8);
+  expect(casc32, 1, 256, 128, 1, 1);
+  // the round is that of the device's CUs
+  expect(mrt64, 0, 256, 128, 3, 11, 32);
+  expect(mrt64, 0, 64, 64, 4, 2, 32);
+  if (!fails) std::printf("RESULT OK\n");
+  return fails != 0;
+}

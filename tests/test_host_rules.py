@@ -36,3 +36,7 @@ def test_checkpoint_count_streams():
 
 def test_cone_kernel_choice(tmp_path):
     run_program(tmp_path, "cone_shape_check")
+
+
+def test_steps_shape(tmp_path):
+    run_program(tmp_path, "steps_shape_check")
