@@ -566,7 +566,9 @@ struct Engine {
   }
   StepsShape steps_shape(int dir) const {
     if (!steps_possible()) return {1, 1};
-    return lbmx::steps_shape(d, dir, (int)bcs.size(), N, cus(), [&](int H) {
+    StepsFields f;
+    f.add(d.nx, d.ny);
+    return lbmx::steps_shape(d, dir, (int)bcs.size(), f, cus(), [&](int H) {
       return (long long)((d.nx + kTileX - 1) / kTileX) * ((d.ny + H - 1) / H);
     });
   }
@@ -582,12 +584,12 @@ struct Engine {
     c.m = params();
     c.obj = obj;
   }
-  // forward steps t, t + 1, .. from src in one launch; the state after the j-th goes to dst[j]
+  // forward steps t, t + 1, .. from src in one launch (tiles of H rows); the state after the j-th goes to dst[j]
   // (null: not kept; the last always is)
-  hipError_t run_fwd_steps(const void* src, void* const* dst, int t, int K, bool with_obj) {
+  hipError_t run_fwd_steps(const void* src, void* const* dst, int t, int K, int H, bool with_obj) {
     if (K == 1) return run_fwd(fwd_args(src, dst[0], t, with_obj));
     FwdSteps a{};
-    fill_steps(a.c, K, steps_shape(0).H);
+    fill_steps(a.c, K, H);
     a.c.obj.acc = (with_obj && obj_set && obj.nterm > 0) ? static_cast<double*>(acc_dev.p) : nullptr;
     a.src = src;
     a.t = t;
@@ -606,10 +608,10 @@ struct Engine {
 #undef CALL
   }
   // reverse steps t, t - 1, .. in one launch; state[j] = p_{t-j-1}
-  hipError_t run_adj_steps(void* const* state, const void* lin, void* lout, int t, int K, const ObjArgs& oa) {
+  hipError_t run_adj_steps(void* const* state, const void* lin, void* lout, int t, int K, int H, const ObjArgs& oa) {
     if (K == 1) return run_adj(adj_args(state[0], lin, lout, t, oa));
     AdjSteps a{};
-    fill_steps(a.c, K, steps_shape(1).H);
+    fill_steps(a.c, K, H);
     a.c.obj = oa;
     a.c.obj.acc = nullptr;
     a.lam_in = lin;
@@ -753,12 +755,12 @@ struct Engine {
   // the launches of nsteps forward steps from the current state; the last step by itself: its
   // input p_{t-1} stays available
   void advance(int nsteps, bool with_obj) {
-    const int most = steps_shape(0).K;
+    const StepsShape sh = steps_shape(0);
     for (int left = nsteps; left > 0;) {
-      const int k = left == 1 ? 1 : std::min(left - 1, most);
+      const int k = left == 1 ? 1 : std::min(left - 1, sh.K);
       void* dst[kMaxSteps] = {};
       dst[k - 1] = prev;
-      HIP_OK(run_fwd_steps(cur, dst, t + 1, k, with_obj));
+      HIP_OK(run_fwd_steps(cur, dst, t + 1, k, sh.H, with_obj));
       std::swap(cur, prev);
       t += k;
       left -= k;
@@ -847,9 +849,9 @@ struct Engine {
     oa.acc = nullptr;
     if (!with_obj) oa.nterm = 0;
 
+    const StepsShape sh[2] = {steps_shape(0), steps_shape(1)};
     const SweepLaunches plan =
-        plan_launches(nsteps, naive, slotbuf, pool[0]->p, pool[1]->p, with_obj, ckpt_mode, steps_shape(0).K,
-                      steps_shape(1).K);
+        plan_launches(nsteps, naive, slotbuf, pool[0]->p, pool[1]->p, with_obj, ckpt_mode, sh[0].K, sh[1].K);
     const PassResult& pr = plan.result;
     auto tf0 = std::chrono::steady_clock::now();
     std::chrono::steady_clock::time_point t_fwd_end;
@@ -867,7 +869,7 @@ struct Engine {
           break;
         }
         case SweepOp::kFwd:
-          HIP_OK(run_fwd_steps(plan.buffers[g.src], bufs, g.t, g.steps(), g.with_obj));
+          HIP_OK(run_fwd_steps(plan.buffers[g.src], bufs, g.t, g.steps(), sh[0].H, g.with_obj));
           break;
         case SweepOp::kAdj: {
           if (!reverse_started) {
@@ -877,7 +879,7 @@ struct Engine {
             zero_async(lam_a.p, lam_bytes(), stream);
             zero_async(sens_dev.p, (size_t)N * 8, stream);
           }
-          HIP_OK(run_adj_steps(bufs, lin, lout, g.t, g.steps(), oa));
+          HIP_OK(run_adj_steps(bufs, lin, lout, g.t, g.steps(), sh[1].H, oa));
           std::swap(lin, lout);
           break;
         }
@@ -1039,12 +1041,12 @@ struct Engine {
       void* lin = lam_a.p;
       void* lout = lam_b.p;
       HIP_OK(hipEventRecord(e0, stream));
-      const int most = steps_shape(1).K;
+      const StepsShape sh = steps_shape(1);
       for (int left = nsweeps; left > 0;) {
-        const int k = std::min(left, most);
+        const int k = std::min(left, sh.K);
         void* state[kMaxSteps];
         std::fill(state, state + k, cur);
-        HIP_OK(run_adj_steps(state, lin, lout, std::max(1, t), k, oa));
+        HIP_OK(run_adj_steps(state, lin, lout, std::max(1, t), k, sh.H, oa));
         std::swap(lin, lout);
         left -= k;
       }
@@ -1180,13 +1182,13 @@ struct Batch {
   // steps per launch and tile rows of a gradient pass (dir: 0 forward, 1 reverse)
   StepsShape shape_of(int dir) const {
     if (tile_set || !m[0]->steps_possible()) return {1, 1};
-    long long nodes = 0;
+    StepsFields f;
     size_t pieces = 0;
     for (const Engine* e : m) {
-      nodes += e->N;
+      f.add(e->d.nx, e->d.ny);
       pieces = std::max(pieces, e->bcs.size());
     }
-    return lbmx::steps_shape(m[0]->d, dir, (int)pieces, nodes, m[0]->cus(), [&](int H) {
+    return lbmx::steps_shape(m[0]->d, dir, (int)pieces, f, m[0]->cus(), [&](int H) {
       long long n = 0;
       for (const Engine* e : m) n += (long long)((e->d.nx + kTileX - 1) / kTileX) * ((e->d.ny + H - 1) / H);
       return n;

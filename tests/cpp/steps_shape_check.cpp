@@ -19,7 +19,9 @@ static StepsShape shape(const Form& f, int dir, int nx, int ny, int nbc = 7, int
   d.collision = f.collision;
   d.design = f.design;
   d.precision = f.precision;
-  return steps_shape(d, dir, nbc, (long long)nx * ny, cus, [&](int H) {
+  StepsFields fields;
+  fields.add(nx, ny);
+  return steps_shape(d, dir, nbc, fields, cus, [&](int H) {
     return (long long)((nx + kTileX - 1) / kTileX) * ((ny + H - 1) / H);
   });
 }
@@ -68,6 +70,46 @@ int main() {
   // the round is that of the device's CUs
   expect(mrt64, 0, 256, 128, 3, 11, 32);
   expect(mrt64, 0, 64, 64, 4, 2, 32);
+  // several rounds: two workgroups of the D2Q9 FP32 forward sweep share a CU
+  const Form casc64{LBMX_D2Q9, LBMX_CASCADED, LBMX_DESIGN_PBB, LBMX_FP64};
+  expect(casc64, 0, 1024, 512, 3, 11);
+  expect(casc64, 0, 200, 1600, 2, 13);
+  const Form mrt32{LBMX_D2Q9, LBMX_MRT, LBMX_DESIGN_BRINKMAN, LBMX_FP32};
+  const Form mrt16{LBMX_D2Q9, LBMX_MRT, LBMX_DESIGN_PBB, LBMX_BF16_SHIFTED};
+  const Form th64{LBMX_D2Q9_D2Q5, LBMX_MRT, LBMX_DESIGN_PBB, LBMX_FP64};
+  const Form th32{LBMX_D2Q9_D2Q5, LBMX_MRT, LBMX_DESIGN_BRINKMAN, LBMX_FP32};
+  expect(mrt64, 0, 1024, 512, 3, 11);
+  expect(mrt64, 1, 1024, 512, 3, 7);
+  expect(mrt32, 0, 1024, 512, 3, 7);
+  expect(mrt32, 1, 1024, 512, 3, 11);
+  expect(th64, 0, 1024, 512, 2, 13);
+  expect(th64, 1, 1024, 512, 3, 6);
+  expect(casc32, 0, 600, 400, 3, 7);
+  expect(casc32, 0, 1280, 640, 3, 7);
+  expect(casc32, 0, 2048, 1024, 1, 1);
+  // narrow fields: fewer steps or one, unless there are few rounds
+  expect(th32, 0, 2048, 1024, 3, 11);
+  expect(th32, 0, 128, 8000, 2, 9);
+  expect(th32, 0, 65, 2400, 3, 11);
+  expect(mrt32, 0, 200, 6000, 1, 1);
+  expect(mrt32, 0, 200, 1600, 3, 7);
+  expect(mrt32, 1, 200, 1600, 1, 1);
+  expect(mrt32, 1, 100, 2400, 3, 11);
+  expect(mrt64, 0, 65, 16000, 3, 11);
+  expect(mrt64, 1, 65, 16000, 1, 1);
+  expect(mrt64, 1, 200, 1600, 3, 7);
+  expect(mrt16, 1, 128, 8000, 1, 1);
+  expect(mrt16, 1, 520, 2200, 3, 11);
+  expect(th64, 1, 128, 8000, 2, 9);
+  expect(th64, 1, 65, 2400, 1, 1);
+  expect(th64, 1, 64, 3000, 1, 1);
+  expect(mrt32, 1, 64, 4000, 3, 11);
+  expect(th64, 1, 512, 300, 3, 6);
+  expect(th64, 0, 64, 4000, 1, 1);
+  expect(th64, 0, 64, 6000, 2, 13);
+  expect(mrt64, 1, 64, 4000, 1, 1);
+  expect(mrt64, 0, 64, 4000, 3, 11);
+  expect(mrt32, 1, 64, 16000, 1, 1);
   if (!fails) std::printf("RESULT OK\n");
   return fails != 0;
 }
