@@ -45,26 +45,16 @@ struct StepsNode {
 // (each wave copies what it reads itself; waves that copy the same piece write the same words).
 template <class L>
 __device__ __forceinline__ StepsNode steps_node(const StepsCommon& c, int x0, int y0, const double* tf, int tf_stride) {
-  const int h = c.K - 1, rows = c.H + 2 * h, pitch = kTileX + 2 * h;
+  const int h = c.K - 1;
   const int lane = (int)threadIdx.x, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+  const StepsPlace p = steps_place(c.K, c.H, wave, lane);
   StepsNode n;
-  int dx = lane, dy = wave - h;
-  n.row = wave >= h && wave < h + c.H;
-  bool held = true;
-  const bool side = wave >= rows;
-  if (side) {
-    const int i = (wave - rows) * kTileX + lane, r = i / (2 * h), k = i - r * (2 * h);
-    dx = k < h ? k - h : kTileX + k - h;
-    dy = r - h;
-    held = r < rows;
-  }
-  n.x = x0 + dx;
-  n.y = y0 + dy;
-  n.active = held && n.x >= 0 && n.x < c.nx && n.y >= 0 && n.y < c.ny;
-  const int ox = dx < 0 ? -dx : (dx >= kTileX ? dx - kTileX + 1 : 0);
-  const int oy = dy < 0 ? -dy : (dy >= c.H ? dy - c.H + 1 : 0);
-  n.ring = ox > oy ? ox : oy;
-  n.cell = (dy + h) * pitch + dx + h;
+  n.row = p.row;
+  n.x = x0 + p.dx;
+  n.y = y0 + p.dy;
+  n.active = p.held && n.x >= 0 && n.x < c.nx && n.y >= 0 && n.y < c.ny;
+  n.ring = p.ring;
+  n.cell = p.cell;
   n.off = n.active ? layout_off(c.ls, n.x, n.y, 0) : 0u;
   n.bnd = n.active && on_boundary<L>(n.x, n.y, 0, c.nx, c.ny, 1);
   n.pieces = 0;
@@ -72,12 +62,13 @@ __device__ __forceinline__ StepsNode steps_node(const StepsCommon& c, int x0, in
     bool meets = false;
     if (lane < c.nbc) {
       const int* b = c.bcs[lane].box;
-      const int xa = side ? x0 - h : x0, xb = side ? x0 + kTileX - 1 + h : x0 + kTileX - 1;
-      const int ya = side ? y0 - h : y0 + dy, yb = side ? y0 + c.H - 1 + h : y0 + dy;
+      const int xa = p.side ? x0 - h : x0, xb = p.side ? x0 + kTileX - 1 + h : x0 + kTileX - 1;
+      const int ya = p.side ? y0 - h : y0 + p.dy, yb = p.side ? y0 + c.H - 1 + h : y0 + p.dy;
       meets = (b[0] <= xb) & (b[1] >= xa) & (b[2] <= yb) & (b[3] >= ya);
     }
     n.pieces = __ballot(meets);
     constexpr int W = (int)(sizeof(DevBC) / 4);
+    static_assert(sizeof(DevBC) % 8 == 0 && W + kMaxSteps <= kTileX, "a lane copies one word or one time factor");
     const unsigned int* s = reinterpret_cast<const unsigned int*>(c.bcs);
     unsigned int* d = reinterpret_cast<unsigned int*>(pieces_lds);
     double* t = reinterpret_cast<double*>(pieces_lds + (size_t)c.nbc * sizeof(DevBC));

@@ -20,6 +20,30 @@ constexpr int steps_waves(int K, int H) {
   const int rows = H + 2 * (K - 1), side = 2 * (K - 1) * rows;
   return rows + (side + kTileX - 1) / kTileX;
 }
+// Where a lane's node lies: offsets from the tile's first node, distance from the tile (0 inside)
+// and LDS cell. One wave holds one row of the region, x0 .. x0 + 63; the ring's columns beside
+// those 64 are packed into further waves, whose last lanes hold nothing.
+struct StepsPlace {
+  int dx, dy, ring, cell;
+  bool row;   // the wave holds a row of the tile (not of its ring)
+  bool side;  // the wave holds columns beside the 64
+  bool held;
+};
+constexpr StepsPlace steps_place(int K, int H, int wave, int lane) {
+  const int h = K - 1, rows = H + 2 * h, pitch = kTileX + 2 * h;
+  StepsPlace p{lane, wave - h, 0, 0, wave >= h && wave < h + H, wave >= rows, true};
+  if (p.side) {
+    const int i = (wave - rows) * kTileX + lane, r = i / (2 * h), k = i - r * (2 * h);
+    p.dx = k < h ? k - h : kTileX + k - h;
+    p.dy = r - h;
+    p.held = r < rows;
+  }
+  const int ox = p.dx < 0 ? -p.dx : (p.dx >= kTileX ? p.dx - kTileX + 1 : 0);
+  const int oy = p.dy < 0 ? -p.dy : (p.dy >= H ? p.dy - H + 1 : 0);
+  p.ring = ox > oy ? ox : oy;
+  p.cell = (p.dy + h) * pitch + p.dx + h;
+  return p;
+}
 // Most waves of a workgroup. The FP64 reverse steps need more than the 128 registers that a
 // workgroup of 16 waves leaves each lane (they spill up to 200 of them, and at 1024 x 512 a
 // reverse step takes 30 us instead of the single-step sweep's 27); with 12 waves they have 168

@@ -34,7 +34,64 @@ static void expect(const Form& f, int dir, int nx, int ny, int K, int H, int cus
   ++fails;
 }
 
+// Every LDS access of a launch of K steps on tiles of H rows lies inside its region, and every
+// cell of the region has one lane.
+static void check_places(int K, int H) {
+  const int h = K - 1, rows = H + 2 * h, pitch = kTileX + 2 * h, cells = steps_cells(K, H);
+  std::vector<int> held(cells, 0), ring(cells, -1);
+  auto fail = [&](const char* what, int wave, int lane) {
+    std::printf("K %d H %d wave %d lane %d: %s\n", K, H, wave, lane, what);
+    ++fails;
+  };
+  for (int wave = 0; wave < steps_waves(K, H); ++wave)
+    for (int lane = 0; lane < kTileX; ++lane) {
+      const StepsPlace p = steps_place(K, H, wave, lane);
+      if (!p.held) {
+        if (!p.side || wave + 1 != steps_waves(K, H)) fail("holds nothing", wave, lane);
+        continue;
+      }
+      if (p.cell < 0 || p.cell >= cells) {
+        fail("cell out of range", wave, lane);
+        continue;
+      }
+      if (p.ring < 0 || p.ring > h) fail("beyond the ring", wave, lane);
+      if (p.row && (p.side || p.dx != lane || p.dy < 0 || p.dy >= H)) fail("not a row of the tile", wave, lane);
+      ++held[p.cell];
+      ring[p.cell] = p.ring;
+      // step j is taken by ring <= K - j; it reads the cells around its own from step j - 1, and
+      // writes reflections around it for step j + 1 where ring <= K - j - 1
+      if (p.ring < h)
+        for (int y = p.dy - 1; y <= p.dy + 1; ++y)
+          for (int x = p.dx - 1; x <= p.dx + 1; ++x) {
+            if (x < -h || x >= kTileX + h || y < -h || y >= H + h) fail("neighbour outside the region", wave, lane);
+            const int at = p.cell + (x - p.dx) + (y - p.dy) * pitch;
+            if (at != (y + h) * pitch + x + h || at < 0 || at >= cells) fail("neighbour's cell", wave, lane);
+          }
+    }
+  for (int c = 0; c < cells; ++c)
+    if (held[c] != 1) fail("a cell without one lane", c / pitch, c % pitch);
+  for (int y = 0; y < rows; ++y)  // a node of ring r finds its neighbours' values of the step before
+    for (int x = 0; x < pitch; ++x)
+      for (int dy = -1; dy <= 1; ++dy)
+        for (int dx = -1; dx <= 1; ++dx)
+          if (ring[y * pitch + x] < h && ring[(y + dy) * pitch + x + dx] > ring[y * pitch + x] + 1)
+            fail("a neighbour two rings out", y, x);
+  for (int nbc = 0; nbc <= kMaxBC; ++nbc) {
+    const size_t bytes = steps_pieces_bytes(nbc, K);
+    if (bytes % 16 || (size_t)nbc * sizeof(DevBC) % sizeof(double) ||
+        (size_t)nbc * sizeof(DevBC) + (size_t)K * nbc * sizeof(double) > bytes)
+      fail("pieces and time factors", nbc, 0);
+  }
+  for (int Q : {9, 14})
+    for (int elem : {2, 4, 8}) {
+      const size_t field = ((size_t)cells * Q * elem + 15) & ~(size_t)15;  // the second field's offset
+      if (field % elem || (K > 2 ? 2 : 1) * field > steps_field_bytes(K, H, Q, elem)) fail("fields", Q, elem);
+    }
+}
+
 int main() {
+  for (int K = 2; K <= kMaxSteps; ++K)
+    for (int H = 2; steps_waves(K, H) <= 16; ++H) check_places(K, H);
   std::vector<Form> forms;
   for (int lat : {LBMX_D2Q9, LBMX_D2Q9_D2Q5})
     for (int coll : {LBMX_BGK, LBMX_MRT, LBMX_CASCADED})
