@@ -98,7 +98,8 @@ struct StepsFields {
 // the thermal FP64 reverse sweep (64x3000 1.16).
 // The single-step sweeps also stay where the arithmetic of the rings costs more than the saved
 // passes: the 16-bit forward sweeps, which compute two nodes per lane (D2Q9 1024x512, in a gradient
-// pass that keeps every state, 8.4 and 9.5, 1536x512 12.2 and 13.9), the cascaded FP32 forward
+// pass that keeps every state, wall time of one box, 8.4 and 9.5, 1536x512 12.2 and 13.9; a kernel
+// trace of passes that recompute gives 9.4 for the former), the cascaded FP32 forward
 // sweep above 2^20 nodes (a gradient pass that keeps every state: 330x3600 1.12 of single steps,
 // 2048x1024 1.04, 1280x640 0.93), and the thermal FP64 reverse sweep with Brinkman's term, which
 // spills (640x300 21.4 and 23.0).
